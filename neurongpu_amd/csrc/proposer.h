@@ -60,12 +60,14 @@ constexpr int kPropPkBytes = kPropPkB3 + 16;
 
 // Training on logged samples (proposer.hip): minibatches of `batch` samples
 // drawn with Philox from [0, n), mean squared error, SGD or Adam.
+constexpr int kPropGradRow = kPropNParam + 1;  // gradients and the loss
+constexpr int kPropGradRows = 256;             // most blocks of a minibatch
 struct PropTrainArgs {
   const float *samples;        // [n][kPropSample]
   unsigned long long n;
   float *w;                    // FP32 master weights
-  float *grad;                 // [kPropNParam] accumulated gradient
-  float *loss;                 // [1] accumulated loss
+  float *grad;                 // [kPropGradRows][kPropGradRow] partial sums
+  float *loss;                 // [1] the minibatch's summed loss
   float *m, *v;                // Adam moments
   uint16_t *w_bf16;            // inference copy
   int batch;

@@ -77,6 +77,35 @@ def test_training_step_matches_numpy(ngpu):
     assert np.allclose(w1, want, rtol=1e-4, atol=2e-6)
 
 
+@pytest.mark.parametrize("batch", [1, 31, 32, 33, 127, 129, 8191, 40001])
+def test_training_step_at_tile_edges(ngpu, batch):
+    """The full-batch SGD step and its loss at batch sizes around the 32-
+    sample tiles and the 128-sample blocks, and with several tiles per wave,
+    against FP64.  Tolerance: FP32 sums of `batch` terms of either sign,
+    bounded by the sum of their magnitudes."""
+    log("case proposer_tiles", batch)
+    rng = np.random.default_rng(batch)
+    w0 = rng.normal(0.0, 0.3, NP).astype(np.float32)
+    smp = np.zeros((batch, 8), np.float32)
+    smp[:, :NI] = rng.normal(0.0, 1.0, (batch, NI))
+    smp[:, NI] = rng.normal(0.0, 1.0, batch)
+    ngpu.ProposerSetWeights(w0)
+    ngpu.ProposerSetSamples(smp)
+    lr = 0.05
+    loss = ngpu.ProposerTrain(1, batch=batch, lr=lr, adam=False,
+                              full_batch=True)
+    w1 = ngpu.ProposerGetWeights()
+    l_ref, g = mlp_loss_grad(w0, smp[:, :NI].astype(np.float64),
+                             smp[:, NI].astype(np.float64))
+    assert abs(loss - l_ref) <= 1e-5 * l_ref
+    assert np.allclose(w1, w0.astype(np.float64) - lr * g, rtol=1e-6,
+                       atol=2e-6)
+    # a fixed order of summation: a second run gives the same bits
+    ngpu.ProposerSetWeights(w0)
+    ngpu.ProposerTrain(1, batch=batch, lr=lr, adam=False, full_batch=True)
+    assert np.array_equal(w1, ngpu.ProposerGetWeights())
+
+
 def test_training_fits_known_function(ngpu):
     """Adam on samples of t = 0.5 x0 - 0.3 x4 + 0.2 |x1| reaches a mean
     squared error below 2e-3."""
