@@ -1,0 +1,67 @@
+"""The second RK5 pass's lane layouts: neurons on lanes of their own, then
+one neuron per quad of lanes for a wave's last neurons, against the
+single-pass kernel (one neuron a lane to the end of the step), bit for bit.
+"""
+import numpy as np
+import pytest
+
+from neurongpu_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+N = 700
+
+
+def spec(ports, uniform, tol=1e-6):
+    """Spiking AdEx neurons (drive above the rheobase, refractory for 5
+    steps) with recurrent synapses of dyadic weight on every port."""
+    rng = np.random.default_rng(10 * ports + uniform)
+    I_e = 900.0 if uniform else rng.uniform(500.0, 1500.0, N)
+    src = rng.integers(0, N, 20 * N)
+    tgt = rng.integers(0, N, 20 * N)
+    port = rng.integers(0, ports, 20 * N)
+    conns = [{"src": src[port == q], "tgt": tgt[port == q], "weight": 0.25,
+              "delay": 0.1 * rng.integers(1, 8, int((port == q).sum())),
+              "port": q} for q in range(ports)]
+    return {"seed": 3, "conns": conns, "groups": [
+        {"model": "aeif_cond_beta", "n": N, "n_port": ports,
+         "params": {"I_e": I_e, "t_ref": 0.5,
+                    "E_rev": [0.0, -85.0, -10.0, -70.0][:ports],
+                    "tau_rise": [0.5, 0.5, 1.0, 2.0][:ports],
+                    "tau_decay": [2.0, 5.0, 1.0, 4.0][:ports]},
+         "vars": {"V_m": rng.uniform(-70.0, -40.0, N).astype(np.float32)},
+         "rk5": {"rk5_tol": tol}}]}
+
+
+def run(ngpu, sp, settings):
+    groups, _ = wl.build_from_spec(ngpu, sp)
+    ngpu.SetKernelStatus(settings)
+    ngpu.ActivateSpikeCount(groups[0])
+    ngpu.Simulate(60.0)
+    out = [np.array(ngpu.GetNeuronVar(0, N, v))
+           for v in ("V_m", "w", "g", "g1")]
+    out.append(np.array(ngpu.GetNeuronIntVar(0, N, "spike_count")))
+    out.append(ngpu.GetHotPathStats())
+    return out
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ports", [1, 2, 3, 4])
+def test_second_pass_layouts(ngpu, ports, uniform):
+    """Grids of 256 blocks (every list fits the quads), 1 block (64 quads:
+    longer lists run on whole waves first), and binned steps, where the pass
+    overlaps the next step; 4 ports keep one lane per neuron."""
+    print("case second_pass", ports, uniform, flush=True)
+    sp = spec(ports, uniform)
+    want = run(ngpu, sp, {"rk5_two_pass": 0})
+    assert want[4].sum() > 2 * N
+    for st in ({"rk5_pass2_grid": 256}, {"rk5_pass2_grid": 1},
+               {"rk5_pass2_grid": 1, "rk5_budget": 3},
+               {"delivery_mode": 1}, {"delivery_mode": 1,
+                                      "rk5_pass2_grid": 1}):
+        print("  settings", st, flush=True)
+        got = run(ngpu, sp, st)
+        for a, b in zip(want[:5], got[:5]):
+            assert np.array_equal(a, b)
+        # the same attempts, accepted and rejected
+        assert got[5] == want[5]
