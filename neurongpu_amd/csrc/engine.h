@@ -340,8 +340,7 @@ class Engine {
   StepClock *StepClockNext() const { return d_clock.p + (clock_slot ^ 1); }
   void DropGraphs();
   StepClock HostClock() const;  // values of the next step
-  DBuf<uint32_t> d_bin_hist, d_bin_tot, d_bin_bstart, d_bin_cstart,
-      d_bin_meta;
+  DBuf<uint32_t> d_bin_tot, d_bin_cstart, d_bin_meta;
   DBuf<unsigned long long> d_bin_ev;
   DBuf<float> d_bin_part;
   // sets up the binned-delivery buffers; false if the network cannot use it

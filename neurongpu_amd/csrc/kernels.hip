@@ -24,6 +24,8 @@
 //   post STDP       src/rev_spike.cu:41-75, src/stdp.cu:24-51
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ngpu_device.h"
 #include "ngpu_kernels.h"
 #include "proposer.h"
@@ -1225,6 +1227,7 @@ __device__ __forceinline__ DeliveryArgs clocked(const DeliveryArgs &D) {
   DeliveryArgs A = D;
   if (A.clock) {
     A.gs = A.clock->gs;
+    A.slot = (int)(A.gs % A.R);
     A.T = A.clock->T;
   }
   return A;
@@ -1233,9 +1236,16 @@ __device__ __forceinline__ RevArgs clocked(const RevArgs &R) {
   RevArgs A = R;
   if (A.clock) {
     A.gs = A.clock->gs;
+    A.slot = (int)(A.gs % A.R);
     A.T = A.clock->T;
   }
   return A;
+}
+
+// Ring slot of k steps before the step of slot `slot` (0 <= k < R).
+__device__ __forceinline__ int slot_back(int slot, int k, int R) {
+  const int s = slot - k;
+  return s < 0 ? s + R : s;
 }
 
 // Second RK5 pass and the delivery of the same step in one launch: blocks
@@ -1419,7 +1429,7 @@ constexpr int kMaxDelaySlots = 4096;  // checked on the host at calibration
 // counts of slots gs-1-d.  Virtual block 0 also clears the ring counter of
 // the slot the next step fills (slot gs+1 is never read in this step).
 // Returns the number of pairs.  BS: threads per block; s_part holds BS
-// entries.
+// entries and may be used again after the call.
 template <int BS = kBlock>
 __device__ __forceinline__ uint32_t delivery_prologue(const DeliveryArgs &A,
                                                       uint32_t vblock,
@@ -1427,14 +1437,15 @@ __device__ __forceinline__ uint32_t delivery_prologue(const DeliveryArgs &A,
                                                       uint32_t *s_part) {
   const int D = A.D;
   const int tid = threadIdx.x;
+  // spikes of delay slot d due this step (slot gs-1-d; D <= R - 2)
+  auto due = [&](int d) -> uint32_t {
+    return (long long)d < A.gs ? A.ring_n[slot_back(A.slot, d + 1, A.R)] : 0u;
+  };
+  const int next = A.slot + 1 == A.R ? 0 : A.slot + 1;
   if (D <= 64) {
     // one wave: scan of the D counts through cross-lane shuffles
     if (tid < 64) {
-      uint32_t n = 0;
-      if (tid < D) {
-        long long s = A.gs - 1 - tid;
-        if (s >= 0) n = A.ring_n[s % A.R];
-      }
+      const uint32_t n = tid < D ? due(tid) : 0u;
       uint32_t incl = n;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -1445,7 +1456,7 @@ __device__ __forceinline__ uint32_t delivery_prologue(const DeliveryArgs &A,
       if (tid == 63) s_pre[D] = incl;
     }
     __syncthreads();
-    if (vblock == 0 && tid == 0) A.ring_n[(A.gs + 1) % A.R] = 0u;
+    if (vblock == 0 && tid == 0) A.ring_n[next] = 0u;
     return s_pre[D];
   }
   // per-thread partial sums of the due spike counts over d
@@ -1453,12 +1464,7 @@ __device__ __forceinline__ uint32_t delivery_prologue(const DeliveryArgs &A,
   uint32_t run = 0;
   for (int k = 0; k < per; k++) {
     int d = tid * per + k;
-    uint32_t n = 0;
-    if (d < D) {
-      long long s = A.gs - 1 - d;
-      if (s >= 0) n = A.ring_n[s % A.R];
-    }
-    run += n;
+    if (d < D) run += due(d);
   }
   s_part[tid] = run;
   __syncthreads();
@@ -1475,29 +1481,19 @@ __device__ __forceinline__ uint32_t delivery_prologue(const DeliveryArgs &A,
       int d = tid * per + k;
       if (d < D) {
         s_pre[d] = acc;
-        long long s = A.gs - 1 - d;
-        if (s >= 0) acc += A.ring_n[s % A.R];
+        acc += due(d);
       }
     }
     if (tid == BS - 1) s_pre[D] = s_part[BS - 1];
   }
   __syncthreads();
-  if (vblock == 0 && tid == 0) A.ring_n[(A.gs + 1) % A.R] = 0u;
+  if (vblock == 0 && tid == 0) A.ring_n[next] = 0u;
   return s_pre[D];
 }
 
-// Enumerates the synaptic events of this wave's share of the step and calls
-// f(ok, syn, rec, height, mult) for U 64-event chunks at a time (all U
-// record loads are issued before the calls).  The wave takes tiles of pt
-// pairs (the largest power of two in [1, tile_max] that still gives every
-// wave of the virtual grid a tile).  When the tile's segments average at
-// least kLongSegment synapses they are walked one at a time; otherwise
-// the tile's events are spread over the 64 lanes by a lane-level scan of
-// the segment lengths and a binary-lift owner search.  The
-// enumeration depends only on (vblock, vgrid, tile_max) and the ring, so
-// two kernels launched with the same arguments see the same events in the
-// same blocks.  Returns the wave's event count.
-constexpr uint32_t kLongSegment = 32;
+// A wave tile whose segments average at least this many synapses is walked
+// one (spike, delay) pair at a time.
+constexpr uint32_t kLongSegment = 128;
 
 // Synapse segment of (source, delay slot) in the canonical store: its
 // records rec[start .. start + cnt).
@@ -1513,54 +1509,151 @@ struct SegLoc {
   }
 };
 
-// BS: threads per block; Loc(src, d, cnt, start) locates a pair's records
-// in `recs`.
-template <int U, int BS = kBlock, class F, class Loc = SegLoc>
-__device__ __forceinline__ unsigned long long deliver_events(
-    const DeliveryArgs &A, uint32_t vblock, uint32_t vgrid,
-    const uint32_t *s_pre, uint32_t total, F &&f,
-    const unsigned long long *recs = nullptr, Loc loc = Loc{}) {
-  const int D = A.D;
-  if (!recs) recs = A.rec;
-  const uint32_t lane = lane_id();
-  const uint32_t wave = (uint32_t)(vblock * (BS / 64) + threadIdx.x / 64);
-  const uint32_t n_waves = vgrid * (BS / 64);
-  uint32_t pt = (uint32_t)A.tile_max;
-  while (pt > 1 && (total + pt - 1) / pt < n_waves) pt >>= 1;
-  const uint32_t n_tiles = (total + pt - 1) / pt;
-  unsigned long long n_events = 0;
-  for (uint32_t wt = wave; wt < n_tiles; wt += n_waves) {
-    uint32_t pidx = wt * pt + lane;
-    uint32_t cnt = 0, mult = 0;
-    unsigned long long start = 0;
-    float height = 0.0f;
-    if (lane < pt && pidx < total) {
+// A wave's table of the pairs of its tile, in LDS: per pair with synapses
+// the start of its records minus its first event's number in the tile, and
+// the spike's height (WIDE: and multiplicity); and one bit per event of the
+// tile, set for the last event of each pair.  WIDE: records addressed by 64
+// bits, else 32.
+template <bool WIDE>
+struct PairTable {
+  static constexpr int kWords = WIDE ? 64 : 32;   // 64 events each
+  struct Wide {
+    unsigned long long start;
+    float height;
+    uint32_t mult;
+  };
+  struct Narrow {
+    uint32_t start;
+    float height;
+  };
+  typename std::conditional<WIDE, Wide, Narrow>::type pair[64];
+  unsigned long long last[kWords];
+};
+static_assert(sizeof(PairTable<false>) * (kTiledBlock / 64) == kTiledScratch,
+              "LDS of a tiled block");
+
+// Inclusive sum over the wave by DPP (row shifts, then the row totals
+// broadcast), without the LDS latency of shuffles.
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v) {
+#define NGPU_DPP_ADD(ctrl, rows)                                          \
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF,  \
+                                             false)
+  NGPU_DPP_ADD(0x111, 0xF);   // row_shr:1
+  NGPU_DPP_ADD(0x112, 0xF);   // row_shr:2
+  NGPU_DPP_ADD(0x114, 0xF);   // row_shr:4
+  NGPU_DPP_ADD(0x118, 0xF);   // row_shr:8
+  NGPU_DPP_ADD(0x142, 0xA);   // row_bcast:15 into rows 1 and 3
+  NGPU_DPP_ADD(0x143, 0xC);   // row_bcast:31 into rows 2 and 3
+#undef NGPU_DPP_ADD
+  return v;
+}
+
+// Orders a wave's LDS writes before its lanes' later reads (LDS operations
+// of a wave run in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The waves of the virtual grid take equal numbers of wave tiles of pt
+// (spike, delay) pairs, pt at most tile_max.  Tile wt takes the pairs wt, wt
+// + n_tiles, wt + 2 n_tiles, ...: pairs are numbered by delay slot, and a
+// network's delays are rarely uniform, so that runs of consecutive pairs
+// would differ in events many times over (1e6 neurons with normal delays:
+// from 0 to over 8192 events per 8-wave block, scatter 47 us; with strided
+// pairs 22 us).
+//
+// Plastic networks (not STRIDED) keep runs of consecutive pairs, of the
+// largest power of two that still gives every wave a tile: their weights
+// are not dyadic, so the order of the additions into an accumulator decides
+// the last bit of its sum, and a spiking network amplifies it; this order
+// keeps their runs as reproducible as the atomics allow (strided pairs would
+// take 1 us off the 12 us delivery of 2e5 neurons).
+template <bool STRIDED>
+struct TileSplit {
+  uint32_t total, pt, n_tiles, wave, n_waves;
+  __device__ __forceinline__ uint32_t pair(uint32_t wt, uint32_t lane) const {
+    return STRIDED ? lane * n_tiles + wt : wt * pt + lane;
+  }
+  template <int BS>
+  static __device__ __forceinline__ TileSplit make(uint32_t total,
+                                                   uint32_t tile_max,
+                                                   uint32_t vblock,
+                                                   uint32_t vgrid) {
+    TileSplit t;
+    t.total = total;
+    t.wave = vblock * (BS / 64) + threadIdx.x / 64;
+    t.n_waves = vgrid * (BS / 64);
+    if (!STRIDED) {
+      t.pt = 1u << (31 - __clz((int)tile_max));
+      while (t.pt > 1 && (total + t.pt - 1) / t.pt < t.n_waves) t.pt >>= 1;
+      t.n_tiles = (total + t.pt - 1) / t.pt;
+      return t;
+    }
+    const uint32_t all = t.n_waves * tile_max;
+    const uint32_t turns = total > all ? (total + all - 1) / all : 1u;
+    t.pt = (total + t.n_waves * turns - 1) / (t.n_waves * turns);
+    if (t.pt == 0u) t.pt = 1u;
+    t.n_tiles = (total + t.pt - 1) / t.pt;
+    return t;
+  }
+};
+
+// One wave tile: the pairs of its lanes, and their events spread over the
+// wave.  emit() calls f(ok, e, syn, rec, height, mult) for 64 events at a
+// time (e: the event's number in the tile), in groups of U: the records of a
+// group are loaded while the group before it is handed to f.  A lane finds
+// its event's pair by counting the pairs that end before the event (the
+// running count of the groups before, plus the set bits below its own in
+// the group's 64-bit mask) and reads the pair's table entry: two LDS reads
+// and a few VALU instructions per 64 events, where a search of the prefix by
+// cross-lane reads took 11 of them.  Tiles of long segments (kLongSegment
+// on average, or more events than the mask holds) are walked one pair at a
+// time.
+template <int U, bool WIDE>
+struct WaveTile {
+  uint32_t cnt = 0, incl = 0, mult = 0, E = 0;
+  unsigned long long start = 0, nz = 0;
+  float height = 0.0f;
+
+  template <bool STRIDED, class Loc>
+  __device__ __forceinline__ void fetch(const DeliveryArgs &A,
+                                        const TileSplit<STRIDED> &t,
+                                        uint32_t wt,
+                                        const uint32_t *s_pre,
+                                        const Loc &loc) {
+    const uint32_t lane = lane_id();
+    const uint32_t pidx = t.pair(wt, lane);
+    cnt = 0;
+    if (lane < t.pt && pidx < t.total) {
       // delay slot d of this pair: last d with s_pre[d] <= pidx
-      int lo = 0, hi = D;  // s_pre[lo] <= pidx < s_pre[hi]
-      while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (s_pre[mid] <= pidx) lo = mid; else hi = mid;
+      int d = 0, hi = A.D;  // s_pre[d] <= pidx < s_pre[hi]
+      while (hi - d > 1) {
+        const int mid = (d + hi) >> 1;
+        if (s_pre[mid] <= pidx) d = mid; else hi = mid;
       }
-      int d = lo;
-      long long slot = (A.gs - 1 - d) % A.R;
-      long long e = slot * A.cap + (pidx - s_pre[d]);
-      uint32_t src = A.ring_src[e];
+      const long long e =
+          (long long)slot_back(A.slot, d + 1, A.R) * A.cap + (pidx - s_pre[d]);
+      const uint32_t src = A.ring_src[e];
       height = A.ring_h[e];
-      mult = A.ring_cnt[e];
+      if (WIDE) mult = A.ring_cnt[e];
       loc(A, src, d, cnt, start);
     }
-    // exclusive scan of cnt over the wavefront
-    uint32_t incl = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      uint32_t v = __shfl_up(incl, off);
-      if ((int)lane >= off) incl += v;
-    }
-    uint32_t pre = incl - cnt;
-    uint32_t E = __shfl(incl, 63);
-    n_events += E;
-    const unsigned long long nz = __ballot(cnt > 0u);
-    if (E >= (uint32_t)kLongSegment * (uint32_t)__popcll(nz)) {
+    incl = wave_incl_sum(cnt);
+    E = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    nz = __ballot(cnt > 0u);
+  }
+
+  template <class F>
+  __device__ __forceinline__ void emit(PairTable<WIDE> &tab,
+                                       const unsigned long long *recs,
+                                       F &&f) const {
+    if (E == 0u) return;
+    const uint32_t lane = lane_id();
+    const uint32_t pre = incl - cnt;
+    if (E > 64u * PairTable<WIDE>::kWords ||
+        E >= kLongSegment * (uint32_t)__popcll(nz)) {
       // Long segments: one pair at a time, its data broadcast through
       // scalar registers, consecutive lanes on consecutive records.
       unsigned long long m = nz;
@@ -1568,6 +1661,7 @@ __device__ __forceinline__ unsigned long long deliver_events(
         const int j = __ffsll((unsigned long long)m) - 1;
         m &= m - 1ull;
         const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cnt, j);
+        const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)pre, j);
         const uint32_t slo =
             (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)start, j);
         const uint32_t shi =
@@ -1587,42 +1681,112 @@ __device__ __forceinline__ unsigned long long deliver_events(
             r[u] = ok[u] ? recs[syn[u]] : 0ull;
           }
 #pragma unroll
-          for (int u = 0; u < U; u++) f(ok[u], syn[u], r[u], h, mu);
+          for (int u = 0; u < U; u++)
+            f(ok[u], pj + o + 64u * u + lane, syn[u], r[u], h, mu);
         }
       }
-      continue;
+      return;
     }
-    // Short segments: the tile's events are spread over the lanes; each
-    // lane finds its pair by a binary lift over the exclusive scan.
-    for (uint32_t e0 = 0; e0 < E; e0 += 64u * U) {
-      unsigned long long syn[U], r[U];
-      float hj[U];
-      uint32_t mj[U];
-      bool ok[U];
+    // the tile's table (every lane has read the one before: its last group
+    // was handed over)
+    if (lane < (E + 63u) / 64u) tab.last[lane] = 0ull;
+    wave_lds_fence();
+    if (cnt > 0u) {
+      const uint32_t k = lanes_below(nz);
+      tab.pair[k].height = height;
+      if constexpr (WIDE) {
+        tab.pair[k].start = start - pre;
+        tab.pair[k].mult = mult;
+      } else {
+        tab.pair[k].start = (uint32_t)start - pre;
+      }
+      const uint32_t end = incl - 1u;
+      atomicOr(reinterpret_cast<uint32_t *>(tab.last) + (end >> 5),
+               1u << (end & 31u));
+    }
+    wave_lds_fence();
+    struct Group {
+      unsigned long long r[U];
+      unsigned long long syn[U];
+      float h[U];
+      uint32_t m[U];
+    };
+    uint32_t before = 0;   // pairs that end before the next group
+    auto load = [&](Group &g, uint32_t e0) {
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        uint32_t e = e0 + 64u * u + lane;
-        // owner lane j < pt: last lane with pre[j] <= e
-        int j = 0;
-        for (uint32_t stp = pt >> 1; stp > 0; stp >>= 1) {
-          int cand = j + (int)stp;
-          uint32_t pv = __shfl(pre, cand);
-          if (pv <= e) j = cand;
+        const uint32_t w = e0 / 64u + u;
+        // (words past the tile's events are not read)
+        const unsigned long long m64 = 64u * w < E ? tab.last[w] : 0ull;
+        const uint32_t lo = (uint32_t)m64, hi = (uint32_t)(m64 >> 32);
+        const uint32_t k = __builtin_amdgcn_mbcnt_hi(
+            hi, __builtin_amdgcn_mbcnt_lo(lo, before));
+        before += (uint32_t)__popcll(m64);
+        const uint32_t e = 64u * w + lane;
+        const bool ok = e < E;
+        const auto p = tab.pair[ok ? k : 0u];
+        g.h[u] = p.height;
+        if constexpr (WIDE) {
+          g.m[u] = p.mult;
+          g.syn[u] = p.start + e;
+        } else {
+          g.m[u] = 0u;
+          g.syn[u] = (uint32_t)(p.start + e);
         }
-        uint32_t pj = __shfl(pre, j);
-        uint32_t slo = __shfl((uint32_t)start, j);
-        uint32_t shi = __shfl((uint32_t)(start >> 32), j);
-        hj[u] = __shfl(height, j);
-        mj[u] = __shfl(mult, j);
-        ok[u] = e < E;
-        syn[u] = (((unsigned long long)shi << 32) | slo) + (e - pj);
-        r[u] = ok[u] ? recs[syn[u]] : 0ull;
+        g.r[u] = ok ? recs[g.syn[u]] : 0ull;
       }
+    };
+    auto give = [&](const Group &g, uint32_t e0) {
 #pragma unroll
-      for (int u = 0; u < U; u++) f(ok[u], syn[u], r[u], hj[u], mj[u]);
+      for (int u = 0; u < U; u++) {
+        const uint32_t e = e0 + 64u * u + lane;
+        f(e < E, e, g.syn[u], g.r[u], g.h[u], g.m[u]);
+      }
+    };
+    Group ga, gb;
+    load(ga, 0u);
+    for (uint32_t e0 = 0;;) {
+      const bool more_b = e0 + 64u * U < E;
+      if (more_b) load(gb, e0 + 64u * U);
+      give(ga, e0);
+      if (!more_b) break;
+      e0 += 64u * U;
+      const bool more_a = e0 + 64u * U < E;
+      if (more_a) load(ga, e0 + 64u * U);
+      give(gb, e0);
+      if (!more_a) break;
+      e0 += 64u * U;
     }
   }
+};
+
+// Hands the synaptic events of this wave's share of the step to
+// f(ok, e, syn, rec, height, mult); returns their number.  BS: threads per
+// block; tabs: one table per wave of the block; Loc(src, d, cnt, start)
+// locates a pair's records in `recs`.
+template <int U, int BS = kBlock, bool WIDE = true, bool STRIDED = true,
+          class F, class Loc = SegLoc>
+__device__ __forceinline__ unsigned long long deliver_events(
+    const DeliveryArgs &A, uint32_t vblock, uint32_t vgrid,
+    const uint32_t *s_pre, uint32_t total, PairTable<WIDE> *tabs, F &&f,
+    const unsigned long long *recs = nullptr, Loc loc = Loc{}) {
+  if (!recs) recs = A.rec;
+  const TileSplit<STRIDED> t = TileSplit<STRIDED>::template make<BS>(
+      total, (uint32_t)A.tile_max, vblock, vgrid);
+  unsigned long long n_events = 0;
+  for (uint32_t wt = t.wave; wt < t.n_tiles; wt += t.n_waves) {
+    WaveTile<U, WIDE> w;
+    w.fetch(A, t, wt, s_pre, loc);
+    n_events += w.E;
+    w.emit(tabs[threadIdx.x / 64], recs, f);
+  }
   return n_events;
+}
+
+// Accumulator entry of a record's target and port: port * n_total + target,
+// below 20 * 2^26.
+__device__ __forceinline__ uint32_t acc_index(uint32_t tp, long long n_total) {
+  return (tp >> kPortShift) * (uint32_t)n_total + (tp & kTargetMask);
 }
 
 // Dynamic LDS of the delivery kernels: s_pre[D + 1], then (binned
@@ -1638,18 +1802,18 @@ __device__ __forceinline__ void delivery_body(const DeliveryArgs &A,
                                               uint32_t vblock,
                                               uint32_t vgrid) {
   uint32_t *s_pre = s_dyn;
-  __shared__ uint32_t s_part[kBlock];
-  const uint32_t total = delivery_prologue(A, vblock, s_pre, s_part);
-  unsigned long long n_events = deliver_events<2>(
-      A, vblock, vgrid, s_pre, total,
-      [&](bool ok, unsigned long long syn, unsigned long long r, float hj,
-          uint32_t mj) {
+  __shared__ PairTable<true> s_tab[kBlock / 64];
+  const uint32_t total = delivery_prologue(
+      A, vblock, s_pre, reinterpret_cast<uint32_t *>(s_tab));
+  unsigned long long n_events = deliver_events<2, kBlock, true, !PLASTIC>(
+      A, vblock, vgrid, s_pre, total, s_tab,
+      [&](bool ok, uint32_t, unsigned long long syn, unsigned long long r,
+          float hj, uint32_t mj) {
         if (!ok) return;
         uint32_t tp = (uint32_t)r;
         float w = __uint_as_float((uint32_t)(r >> 32));
         uint32_t tgt = tp & kTargetMask;
-        uint32_t port = tp >> kPortShift;
-        unsafeAtomicAdd(A.acc + (long long)port * A.n_total + tgt, hj * w);
+        unsafeAtomicAdd(A.acc + acc_index(tp, A.n_total), hj * w);
         if (PLASTIC) {
           int sgp = A.syn_group[syn];
           if (sgp > 0) {
@@ -1684,27 +1848,25 @@ __global__ __launch_bounds__(kBlock) void delivery_kernel(DeliveryArgs A) {
 // accumulators run at a fixed rate per device whatever the address
 // pattern, so when a step carries many events per accumulator entry the
 // events are first grouped by accumulator range (bin of kBinLen entries):
-//   1 count    per (sub-bin, block) event counts, LDS histogram
-//   2 scan     per sub-bin, exclusive offsets over the blocks, totals
-//   3 scatter  the same enumeration again; each event is written as
-//              (index within bin, value) at its bin's cursor; block 0
-//              also writes the bin and chunk starts.  If the step has more
-//              events than the buffer holds, this phase adds them with
-//              atomics instead and the later phases do nothing.
-//   4 reduce   one block per chunk of events of one bin sums them in LDS
+//   1 scatter  enumerates the events once.  A block keeps its events
+//              (accumulator entry, value) in LDS and counts them per bin;
+//              then it reserves its run in every bin's buffer with one
+//              atomic per bin and writes the events there, and goes on with
+//              its next wave tiles if it has any.  Events beyond a bin's
+//              capacity are added with float atomics instead.
+//   2 reduce   one block per chunk of events of one bin sums them in LDS
 //              (chunk size chosen from the step's event count, see
 //              bin_chunk_size, or one chunk per bin when there are at
 //              least kSingleChunkBins bins of about equal size; then the
-//              sum phase has nothing to do); a bin of one chunk is added to the
-//              accumulators directly, otherwise the partial sums are
+//              sum phase has nothing to do); a bin of one chunk is added to
+//              the accumulators directly, otherwise the partial sums are
 //              written out
-//   5 sum      bins of several chunks: accumulators += sum of partials.
-// Count and scatter use the same grid and tile settings, so every block
-// enumerates the same events in both.
+//   3 sum      bins of several chunks: accumulators += sum of partials;
+//              clears the bins' counts for the next step.
 // ---------------------------------------------------------------------
 
 constexpr int kReduceBlock = 1024;
-constexpr int kBinBlock = 512;  // threads per block of the count and scatter
+constexpr int kBinBlock = 512;  // threads per block of the scatter
 
 // Float add into LDS by compare-and-swap.  On gfx950 the LDS float atomic
 // add runs at about a twelfth of the rate of the integer atomics and of a
@@ -1729,186 +1891,251 @@ __device__ __forceinline__ uint32_t bin_chunk_size(unsigned long long n_ev) {
   return (uint32_t)ch;
 }
 
-// Exclusive scan of val(0..n-1) by one block: out[b] = sum of val(b') for
-// b' < b.  Returns the 64-bit total.  s_part holds kBlock entries.
-template <int BS = kBlock, class F>
-__device__ __forceinline__ unsigned long long block_scan_excl(
-    int n, F val, uint32_t *out, unsigned long long *s_part) {
+// Exclusive scan of val(0..n-1) by one block of BS threads: put(b, sum of
+// val(b') for b' < b).  Returns the total (below 2^32).  s_part: BS / 64
+// entries; the values put are visible to the block after its next barrier.
+template <int BS, class F, class G>
+__device__ __forceinline__ uint32_t block_scan_excl(int n, F val, G put,
+                                                    uint32_t *s_part) {
   const int tid = threadIdx.x;
   const int per = (n + BS - 1) / BS;
-  unsigned long long run = 0;
+  uint32_t run = 0;
   for (int k = 0; k < per; k++) {
-    int b = tid * per + k;
+    const int b = tid * per + k;
     if (b < n) run += val(b);
   }
-  s_part[tid] = run;
+  const uint32_t incl = wave_incl_sum(run);
+  __syncthreads();            // s_part may be in use from a call before
+  if ((tid & 63) == 63) s_part[tid / 64] = incl;
   __syncthreads();
-  for (int off = 1; off < BS; off <<= 1) {
-    unsigned long long v = (tid >= off) ? s_part[tid - off] : 0ull;
-    __syncthreads();
-    s_part[tid] += v;
-    __syncthreads();
+  uint32_t acc = incl - run, total = 0;
+#pragma unroll
+  for (int w = 0; w < BS / 64; w++) {
+    const uint32_t v = s_part[w];
+    acc += w < tid / 64 ? v : 0u;
+    total += v;
   }
-  unsigned long long acc = (tid > 0) ? s_part[tid - 1] : 0ull;
   for (int k = 0; k < per; k++) {
-    int b = tid * per + k;
+    const int b = tid * per + k;
     if (b < n) {
-      unsigned long long v = val(b);  // before out[b]: out may alias the input
-      out[b] = (uint32_t)acc;
+      const uint32_t v = val(b);
+      put(b, acc);
       acc += v;
     }
   }
-  unsigned long long total = s_part[BS - 1];
-  __syncthreads();
   return total;
 }
 
-__global__ __launch_bounds__(kBinBlock) void bin_count_kernel(DeliveryArgs A0,
-                                                              BinArgs B) {
-  const DeliveryArgs A = clocked(A0);
-  uint32_t *s_pre = s_dyn;
-  uint32_t *s_h = s_dyn + A.D + 1;
-  __shared__ uint32_t s_part[kBinBlock];
-  for (int b = threadIdx.x; b < B.nsub; b += kBinBlock) s_h[b] = 0u;
-  const uint32_t total =
-      delivery_prologue<kBinBlock>(A, blockIdx.x, s_pre, s_part);
-  deliver_events<4, kBinBlock>(A, blockIdx.x, gridDim.x, s_pre, total,
-                 [&](bool ok, unsigned long long, unsigned long long r, float,
-                     uint32_t) {
-                   if (!ok) return;
-                   uint32_t tp = (uint32_t)r;
-                   long long idx = (long long)(tp >> kPortShift) * A.n_total +
-                                   (tp & kTargetMask);
-                   atomicAdd(&s_h[idx >> B.sub_shift], 1u);
-                 });
-  __syncthreads();
-  for (int b = threadIdx.x; b < B.nsub; b += kBinBlock)
-    B.hist[(size_t)b * B.grid + blockIdx.x] = s_h[b];
+// LDS of the scatter: events, pair prefix, counts and cursors of the bins.
+inline size_t scatter_lds_bytes(int D, int nb) {
+  return sizeof(unsigned long long) * kBinBuffer +
+         sizeof(uint32_t) * ((size_t)D + 1 + 2 * (size_t)nb);
 }
 
-// one block per sub-bin
-__global__ __launch_bounds__(kBlock) void bin_scan_kernel(BinArgs B) {
-  __shared__ unsigned long long s_part[kBlock];
-  uint32_t *h = B.hist + (size_t)blockIdx.x * B.grid;
-  // in place: each thread reads and rewrites only its own entries
-  unsigned long long t = block_scan_excl(
-      B.grid, [&](int k) -> unsigned long long { return h[k]; }, h, s_part);
-  if (threadIdx.x == 0)
-    B.tot[blockIdx.x] = t > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)t;
-}
-
+// What bounds it: the enumeration's chain of dependent loads (ring entry,
+// segment bounds, records) and the stores to many bins.  A block of 8 waves
+// with room for 8192 events in LDS, two blocks a CU; the host sizes the grid
+// so that a block's events fit its buffer once.  The former version
+// enumerated twice (counts, a scan over the blocks, then the events at
+// their final places).
 __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
     DeliveryArgs A0, BinArgs B) {
   const DeliveryArgs A = clocked(A0);
-  uint32_t *s_pre = s_dyn;
-  uint32_t *s_cur = s_dyn + A.D + 1;
-  __shared__ uint32_t s_part[kBinBlock];
-  __shared__ unsigned long long s_part64[kBinBlock];
-  __shared__ int s_multi;  // some bin has more than one chunk
-  if (threadIdx.x == 0) s_multi = 0;
-  const unsigned long long n_ev = block_scan_excl<kBinBlock>(
-      B.nsub, [&](int b) -> unsigned long long { return B.tot[b]; }, s_cur,
-      s_part64);
-  const bool binned = n_ev <= (unsigned long long)B.ev_cap;
-  if (blockIdx.x == 0) {
-    // bin and chunk starts for the reduce and sum phases; the chunk size
-    // gives about kReduceChunks chunks in all (at least kBinChunkMin
-    // events each), so the reduction fills the device whatever the step's
-    // event count
-    uint32_t ch = bin_chunk_size(n_ev);
-    const int spb = kBinLen >> B.sub_shift;  // sub-bins per bin
-    auto start = [&](int b) -> unsigned long long {
-      return b * spb < B.nsub ? s_cur[b * spb] : n_ev;
-    };
-    // With many bins of about equal size, one chunk per bin: the reduction
-    // still has a block for most CUs, and no partial sums are written and
-    // summed.
-    if (B.nb >= kSingleChunkBins) {
-      unsigned long long mx = 0;
-      for (int b = threadIdx.x; b < B.nb; b += kBinBlock) {
-        const unsigned long long nbin = start(b + 1) - start(b);
-        mx = nbin > mx ? nbin : mx;
+  unsigned long long *s_ev = reinterpret_cast<unsigned long long *>(s_dyn);
+  uint32_t *s_pre = s_dyn + 2 * kBinBuffer;
+  uint32_t *s_cnt = s_pre + A.D + 1;   // events of the round per bin; then
+                                       // the next one's place in the order
+  uint32_t *s_to = s_cnt + B.nb;       // from that place to the bin's buffer
+  __shared__ PairTable<true> s_tab[kBinBlock / 64];
+  __shared__ uint32_t s_part[kBinBlock / 64];
+  __shared__ uint32_t s_n;             // events in the buffer
+  for (int b = threadIdx.x; b < B.nb; b += kBinBlock) s_cnt[b] = 0u;
+  if (threadIdx.x == 0) s_n = 0u;
+  const uint32_t total = delivery_prologue<kBinBlock>(
+      A, blockIdx.x, s_pre, reinterpret_cast<uint32_t *>(s_tab));
+  const TileSplit<true> t = TileSplit<true>::make<kBinBlock>(
+      total, (uint32_t)A.tile_max, blockIdx.x, gridDim.x);
+  unsigned long long n_events = 0;
+  uint32_t wt = t.wave;
+  WaveTile<4, true> w;
+  bool loaded = false;
+  for (;;) {
+    // round: every wave buffers its tiles until one does not fit
+    bool waits = false;
+    while (wt < t.n_tiles && !waits) {
+      if (!loaded) {
+        w.fetch(A, t, wt, s_pre, SegLoc{});
+        n_events += w.E;
+        loaded = true;
       }
-      s_part64[threadIdx.x] = mx;
-      __syncthreads();
-      for (int off = kBinBlock / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < off &&
-            s_part64[threadIdx.x + off] > s_part64[threadIdx.x])
-          s_part64[threadIdx.x] = s_part64[threadIdx.x + off];
-        __syncthreads();
-      }
-      mx = s_part64[0];
-      __syncthreads();
-      if (mx * (unsigned long long)B.nb <= 2ull * n_ev) {
-        const unsigned long long one = (mx + 1023ull) & ~1023ull;
-        if (one > ch && one <= 0x40000000ull) ch = (uint32_t)one;
-      }
-    }
-    for (int b = threadIdx.x; b < B.nb; b += kBinBlock)
-      B.bstart[b] = binned ? (uint32_t)start(b) : 0u;
-    if (threadIdx.x == 0) {
-      B.bstart[B.nb] = binned ? (uint32_t)n_ev : 0u;
-      B.meta[0] = ch;
-    }
-    unsigned long long nc = block_scan_excl<kBinBlock>(
-        B.nb,
-        [&](int b) -> unsigned long long {
-          const unsigned long long c =
-              binned ? (start(b + 1) - start(b) + ch - 1u) / ch : 0u;
-          if (c > 1u) s_multi = 1;
-          return c;
-        },
-        B.cstart, s_part64);
-    if (threadIdx.x == 0) {
-      B.cstart[B.nb] = (uint32_t)nc;
-      B.meta[1] = (uint32_t)s_multi;
-    }
-  }
-  for (int b = threadIdx.x; b < B.nsub; b += kBinBlock)
-    s_cur[b] += B.hist[(size_t)b * B.grid + blockIdx.x];
-  // (the prologue's barriers order these LDS writes before their use)
-  const uint32_t total =
-      delivery_prologue<kBinBlock>(A, blockIdx.x, s_pre, s_part);
-  unsigned long long n_events = deliver_events<4, kBinBlock>(
-      A, blockIdx.x, gridDim.x, s_pre, total,
-      [&](bool ok, unsigned long long, unsigned long long r, float hj,
-          uint32_t) {
-        if (!ok) return;
-        uint32_t tp = (uint32_t)r;
-        float w = __uint_as_float((uint32_t)(r >> 32));
-        long long idx = (long long)(tp >> kPortShift) * A.n_total +
-                        (tp & kTargetMask);
-        float v = hj * w;
-        if (binned) {
-          uint32_t pos = atomicAdd(&s_cur[idx >> B.sub_shift], 1u);
-          B.ev[pos] = ((unsigned long long)__float_as_uint(v) << 32) |
-                      (uint32_t)(idx & (kBinLen - 1));
-        } else {
-          unsafeAtomicAdd(A.acc + idx, v);
+      if (w.E > (uint32_t)kBinBuffer) {
+        // more than any buffer holds: float atomics
+        w.emit(s_tab[threadIdx.x / 64], A.rec,
+               [&](bool ok, uint32_t, unsigned long long,
+                   unsigned long long r, float hj, uint32_t) {
+                 if (ok)
+                   unsafeAtomicAdd(A.acc + acc_index((uint32_t)r, A.n_total),
+                                   hj * __uint_as_float((uint32_t)(r >> 32)));
+               });
+      } else {
+        uint32_t at0 = 0;
+        if (lane_id() == 0) at0 = atomicAdd(&s_n, w.E);
+        at0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)at0);
+        if (at0 + w.E > (uint32_t)kBinBuffer) {
+          // (the places from at0 on stay unused in this round)
+          if (lane_id() == 0) atomicMin(&s_n, at0);
+          waits = true;
+          continue;
         }
-      });
+        w.emit(s_tab[threadIdx.x / 64], A.rec,
+               [&](bool ok, uint32_t e, unsigned long long,
+                   unsigned long long r, float hj, uint32_t) {
+                 if (!ok) return;
+                 const uint32_t idx = acc_index((uint32_t)r, A.n_total);
+                 const float v = hj * __uint_as_float((uint32_t)(r >> 32));
+                 s_ev[at0 + e] =
+                     ((unsigned long long)__float_as_uint(v) << 32) | idx;
+                 atomicAdd(&s_cnt[idx >> kBinShift], 1u);
+               });
+      }
+      loaded = false;
+      wt += t.n_waves;
+    }
+    const int more = __syncthreads_or(waits ? 1 : 0);
+    // reserve the round's runs in the bins' buffers
+    (void)block_scan_excl<kBinBlock>(
+        B.nb, [&](int b) -> uint32_t { return s_cnt[b]; },
+        [&](int b, uint32_t first) {
+          const uint32_t c = s_cnt[b];
+          s_to[b] = (c ? atomicAdd(&B.tot[(size_t)b * kBinStride], c) : 0u) -
+                    first;
+          s_cnt[b] = first;
+        },
+        s_part);
+    const uint32_t n = s_n;
+    __syncthreads();
+    // order the events by bin, in place through registers, so that a bin's
+    // run leaves as whole cache lines
+    constexpr int kPer = kBinBuffer / kBinBlock;
+    unsigned long long ev[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const uint32_t j = k * kBinBlock + threadIdx.x;
+      ev[k] = j < n ? s_ev[j] : 0ull;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+      if (k * kBinBlock + threadIdx.x < n)
+        s_ev[atomicAdd(&s_cnt[(uint32_t)ev[k] >> kBinShift], 1u)] = ev[k];
+    __syncthreads();
+    for (int b = threadIdx.x; b < B.nb; b += kBinBlock) s_cnt[b] = 0u;
+    for (uint32_t j = threadIdx.x; j < n; j += kBinBlock) {
+      const unsigned long long e = s_ev[j];
+      const uint32_t idx = (uint32_t)e, b = idx >> kBinShift;
+      const uint32_t pos = j + s_to[b];
+      if (pos < B.bin_cap)
+        B.ev[(size_t)b * B.bin_cap + pos] =
+            (e & 0xFFFFFFFF00000000ull) | (idx & (kBinLen - 1));
+      else
+        unsafeAtomicAdd(A.acc + idx, __uint_as_float((uint32_t)(e >> 32)));
+    }
+    if (!more) break;
+    __syncthreads();
+    if (threadIdx.x == 0) s_n = 0u;
+    __syncthreads();
+  }
   if (lane_id() == 0 && n_events) {
     atomicAdd(A.events + (blockIdx.x & (kCounterSlots - 1)), n_events);
   }
 }
 
+// Events of bin b in its buffer.
+__device__ __forceinline__ uint32_t bin_events(const BinArgs &B, int b) {
+  const uint32_t n = B.tot[(size_t)b * kBinStride];
+  return n < B.bin_cap ? n : B.bin_cap;
+}
+
 __global__ __launch_bounds__(kReduceBlock) void bin_reduce_kernel(BinArgs B,
                                                                   float *acc) {
   __shared__ float s_a[kBinLen];
-  const uint32_t n_chunk = B.cstart[B.nb];
-  const uint32_t ch = B.meta[0];
+  __shared__ uint32_t s_part[kReduceBlock / 64];
+  __shared__ uint32_t s_red[2][kReduceBlock / 64];
+  __shared__ int s_multi;              // some bin has more than one chunk
+  uint32_t *s_c = s_dyn;               // first chunk of every bin [nb + 1]
+  // events of the step and of the largest bin
+  uint32_t n_ev = 0, mx = 0;
+  for (int b = threadIdx.x; b < B.nb; b += kReduceBlock) {
+    const uint32_t n = bin_events(B, b);
+    n_ev += n;
+    mx = n > mx ? n : mx;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    n_ev += __shfl_xor(n_ev, off);
+    const uint32_t o = __shfl_xor(mx, off);
+    mx = o > mx ? o : mx;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_red[0][threadIdx.x / 64] = n_ev;
+    s_red[1][threadIdx.x / 64] = mx;
+  }
+  if (threadIdx.x == 0) s_multi = 0;
+  __syncthreads();
+  n_ev = mx = 0;
+#pragma unroll
+  for (int w = 0; w < kReduceBlock / 64; w++) {
+    n_ev += s_red[0][w];
+    mx = s_red[1][w] > mx ? s_red[1][w] : mx;
+  }
+  // chunk size: about kReduceChunks chunks in all (at least kBinChunkMin
+  // events each), so that the reduction fills the device whatever the
+  // step's event count; with many bins of about equal size one chunk per
+  // bin: the reduction still has a block for most CUs, and no partial sums
+  // are written and summed
+  uint32_t ch = bin_chunk_size(n_ev);
+  const bool single =
+      B.nb >= kSingleChunkBins &&
+      (unsigned long long)mx * B.nb <= 2ull * n_ev && mx <= 0x40000000u;
+  uint32_t n_chunk = (uint32_t)B.nb;   // chunk b is bin b
+  if (single) {
+    ch = mx;
+  } else {
+    n_chunk = block_scan_excl<kReduceBlock>(
+        B.nb,
+        [&](int b) -> uint32_t {
+          const uint32_t c = (uint32_t)(
+              ((unsigned long long)bin_events(B, b) + ch - 1u) / ch);
+          if (c > 1u) s_multi = 1;
+          return c;
+        },
+        [&](int b, uint32_t first) { s_c[b] = first; }, s_part);
+    if (threadIdx.x == 0) s_c[B.nb] = n_chunk;
+    __syncthreads();
+  }
+  if (blockIdx.x == 0) {     // for the sum phase
+    if (!single)
+      for (int b = threadIdx.x; b <= B.nb; b += kReduceBlock)
+        B.cstart[b] = s_c[b];
+    if (threadIdx.x == 0) B.meta[0] = (uint32_t)s_multi;
+  }
   for (uint32_t w = blockIdx.x; w < n_chunk; w += gridDim.x) {
-    // bin of chunk w: last b with cstart[b] <= w (it has >= 1 chunk)
-    int lo = 0, hi = B.nb;  // cstart[lo] <= w < cstart[hi]
-    while (hi - lo > 1) {
-      int mid = (lo + hi) >> 1;
-      if (B.cstart[mid] <= w) lo = mid; else hi = mid;
+    int b = (int)w;
+    uint32_t k = 0, nc = 1;
+    if (!single) {
+      // bin of chunk w: last b with s_c[b] <= w (it has >= 1 chunk)
+      int lo = 0, hi = B.nb;  // s_c[lo] <= w < s_c[hi]
+      while (hi - lo > 1) {
+        int mid = (lo + hi) >> 1;
+        if (s_c[mid] <= w) lo = mid; else hi = mid;
+      }
+      b = lo;
+      k = w - s_c[b];
+      nc = s_c[b + 1] - s_c[b];
     }
-    const int b = lo;
-    const uint32_t k = w - B.cstart[b];
-    const uint32_t nc = B.cstart[b + 1] - B.cstart[b];
-    const uint32_t e_end = B.bstart[b + 1];
-    const uint32_t e0 = B.bstart[b] + k * ch;
+    const unsigned long long *ev = B.ev + (size_t)b * B.bin_cap;
+    const uint32_t e_end = bin_events(B, b);
+    const uint32_t e0 = k * ch;
     const uint32_t e1 = (e_end - e0 < ch) ? e_end : e0 + ch;
     for (int i = threadIdx.x; i < kBinLen; i += kReduceBlock) s_a[i] = 0.0f;
     __syncthreads();
@@ -1916,14 +2143,14 @@ __global__ __launch_bounds__(kReduceBlock) void bin_reduce_kernel(BinArgs B,
     for (; e + 3u * kReduceBlock < e1; e += 4u * kReduceBlock) {
       unsigned long long v[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = B.ev[e + (uint32_t)u * kReduceBlock];
+      for (int u = 0; u < 4; u++) v[u] = ev[e + (uint32_t)u * kReduceBlock];
 #pragma unroll
       for (int u = 0; u < 4; u++)
         lds_add_f32(&s_a[(uint32_t)v[u]],
                     __uint_as_float((uint32_t)(v[u] >> 32)));
     }
     for (; e < e1; e += kReduceBlock) {
-      unsigned long long v = B.ev[e];
+      unsigned long long v = ev[e];
       lds_add_f32(&s_a[(uint32_t)v], __uint_as_float((uint32_t)(v >> 32)));
     }
     __syncthreads();
@@ -1946,7 +2173,10 @@ __global__ __launch_bounds__(kReduceBlock) void bin_reduce_kernel(BinArgs B,
 __global__ __launch_bounds__(kBlock) void bin_sum_kernel(
     BinArgs B, float *acc, const StepClock *clock, StepClock *clock_next) {
   clock_step(clock, clock_next);
-  if (B.meta[1] == 0u) return;  // every bin was summed by one chunk
+  for (long long b = (long long)blockIdx.x * kBlock + threadIdx.x; b < B.nb;
+       b += (long long)gridDim.x * kBlock)
+    B.tot[b * kBinStride] = 0u;
+  if (B.meta[0] == 0u) return;  // every bin was summed by one chunk
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
        i < B.acc_n; i += (long long)gridDim.x * kBlock) {
     const int b = (int)(i >> kBinShift);
@@ -1987,7 +2217,7 @@ template <bool FIXED>
 __global__ __launch_bounds__(kTiledBlock) void tiled_delivery_kernel(
     DeliveryArgs A0, TileArgs B) {
   const DeliveryArgs A = clocked(A0);
-  __shared__ uint32_t s_part[kTiledBlock];
+  __shared__ PairTable<false> s_tab[kTiledBlock / 64];
   __shared__ int s_big;   // a float atomic went to the accumulator
   // dynamic LDS: the tile (2^tile_shift floats or 64-bit sums), then the
   // pair prefix
@@ -2007,14 +2237,14 @@ __global__ __launch_bounds__(kTiledBlock) void tiled_delivery_kernel(
   if (threadIdx.x == 0) s_big = 0;
   // (the prologue's barriers order the clearing before the first add)
   const uint32_t total =
-      delivery_prologue<kTiledBlock>(A, blockIdx.x, s_pre, s_part);
+      delivery_prologue<kTiledBlock>(A, blockIdx.x, s_pre,
+                                     reinterpret_cast<uint32_t *>(s_tab));
   const long long a0 = (long long)t << B.tile_shift;
-  auto add = [&](bool ok, unsigned long long, unsigned long long r, float hj,
-                 uint32_t) {
+  auto add = [&](bool ok, uint32_t, unsigned long long, unsigned long long r,
+                 float hj, uint32_t) {
     if (!ok) return;
     const uint32_t tp = (uint32_t)r;
-    const long long idx = (long long)(tp >> kPortShift) * A.n_total +
-                          (tp & kTargetMask);
+    const uint32_t idx = acc_index(tp, A.n_total);
     const float v = hj * __uint_as_float((uint32_t)(r >> 32));
     if (FIXED) {
       if (fabsf(hj) <= B.h_max) {
@@ -2030,8 +2260,8 @@ __global__ __launch_bounds__(kTiledBlock) void tiled_delivery_kernel(
     }
   };
   const unsigned long long n_events =
-      deliver_events<4, kTiledBlock, decltype(add) &, TileLoc>(
-          A, k, G, s_pre, total, add, B.trec,
+      deliver_events<4, kTiledBlock, false, true, decltype(add) &, TileLoc>(
+          A, k, G, s_pre, total, s_tab, add, B.trec,
           TileLoc{B.off, (uint32_t)B.T, t});
   __syncthreads();
   const long long lim_ll = B.acc_n - a0;
@@ -2125,9 +2355,8 @@ __global__ __launch_bounds__(kBlock) void rev_kernel(RevArgs A0) {
   // independent (each has this node as its only target), so all 256 lanes
   // walk the reverse index together
   for (int k = 0; k <= A.max_den; k++) {
-    long long s = A.gs - k;
-    if (s < 0) break;
-    long long slot = s % A.R;
+    if (A.gs < k) break;
+    const long long slot = slot_back(A.slot, k, A.R);
     uint32_t n = A.ring_n[slot];
     for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
       uint32_t node = A.ring_src[slot * A.cap + e];
@@ -2160,9 +2389,8 @@ __global__ __launch_bounds__(kBlock) void rev_kernel(RevArgs A0) {
 __global__ __launch_bounds__(kBlock) void den_rev_kernel(RevArgs A0) {
   const RevArgs A = clocked(A0);
   for (int k = 1; k <= A.max_den; k++) {
-    long long s = A.gs - k;
-    if (s < 0) break;
-    long long slot = s % A.R;
+    if (A.gs < k) break;
+    const long long slot = slot_back(A.slot, k, A.R);
     uint32_t n = A.ring_n[slot];
     for (uint32_t e = blockIdx.x * kBlock + threadIdx.x; e < n;
          e += gridDim.x * kBlock) {
@@ -2453,16 +2681,26 @@ void LaunchDeliveryTiled(const DeliveryArgs &a, const TileArgs &b,
 void LaunchDeliveryBinned(const DeliveryArgs &a, const BinArgs &b,
                           int reduce_grid, void *stream) {
   hipStream_t s = (hipStream_t)stream;
-  const size_t lds = delivery_lds_bytes(a.D, b.nsub);
-  hipLaunchKernelGGL(bin_count_kernel, dim3(b.grid), dim3(kBinBlock), lds, s,
-                     a, b);
-  hipLaunchKernelGGL(bin_scan_kernel, dim3(b.nsub), dim3(kBlock), 0, s, b);
-  hipLaunchKernelGGL(bin_scatter_kernel, dim3(b.grid), dim3(kBinBlock), lds, s,
-                     a, b);
+  static bool lds_attr = false;   // both may exceed the default LDS limit
+  if (!lds_attr) {
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void *>(bin_scatter_kernel),
+        hipFuncAttributeMaxDynamicSharedMemorySize,
+        (int)scatter_lds_bytes(kMaxDelaySlots, kMaxBins));
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void *>(bin_reduce_kernel),
+        hipFuncAttributeMaxDynamicSharedMemorySize,
+        (int)(sizeof(uint32_t) * (kMaxBins + 1)));
+    lds_attr = true;
+  }
+  hipLaunchKernelGGL(bin_scatter_kernel, dim3(b.grid), dim3(kBinBlock),
+                     scatter_lds_bytes(a.D, b.nb), s, a, b);
   hipLaunchKernelGGL(bin_reduce_kernel, dim3(reduce_grid), dim3(kReduceBlock),
-                     0, s, b, a.acc);
+                     sizeof(uint32_t) * ((size_t)b.nb + 1), s, b, a.acc);
+  // (with many bins there is rarely anything left to sum: a small grid)
   long long g = (b.acc_n + kBlock - 1) / kBlock;
-  if (g > 2048) g = 2048;
+  const long long most = b.nb >= kSingleChunkBins ? 128 : 512;
+  if (g > most) g = most;
   hipLaunchKernelGGL(bin_sum_kernel, dim3((unsigned)g), dim3(kBlock), 0, s, b,
                      a.acc, a.clock, a.clock_next);
 }

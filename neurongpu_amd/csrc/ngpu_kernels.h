@@ -337,6 +337,7 @@ struct DeliveryArgs {
   long long cap;
   int R;
   long long gs;                 // global step index of this step
+  int slot;                     // its ring slot, gs % R
   int D;                        // number of delay slots (max d_int + 1)
   int tile_max;                 // largest (spike, delay) pairs per wave tile,
                                 // a power of two in [1, 64]
@@ -359,39 +360,32 @@ struct DeliveryArgs {
 };
 
 // Binned delivery (non-plastic networks): the step's synaptic events are
-// counted per (block, accumulator range of kBinLen entries), placed
-// range-major into an event buffer, summed per range in LDS and added to
-// the accumulators once per entry instead of once per event.
+// grouped by accumulator range (bin of kBinLen entries) into one buffer per
+// bin, summed per bin in LDS and added to the accumulators once per entry
+// instead of once per event.
 constexpr int kBinShift = 13;
 constexpr int kBinLen = 1 << kBinShift;   // accumulator entries per bin
-constexpr int kMaxBins = 8192;            // sub-bins a block can count in LDS
-constexpr int kSubBinsTarget = 64;        // preferred largest sub-bin count
+constexpr int kMaxBins = 8192;            // bins a block can count in LDS
+constexpr int kBinBuffer = 8192;          // events a block holds in LDS
+constexpr int kBinStride = 32;            // a bin's counter has a cache line
+                                          // of its own
 constexpr int kReduceChunks = 512;        // target chunk count of a step
 constexpr int kBinChunkMin = 4096;        // fewest events per chunk
 constexpr int kSingleChunkBins = 128;     // from this many bins on, balanced
                                           // bins are reduced in one chunk each
 
 struct BinArgs {
-  // The count and scatter phases group events by sub-bin (2^sub_shift
-  // accumulator entries, at most kBinLen), fine enough that the lanes of a
-  // wavefront rarely hit the same LDS counter; a bin is a run of
-  // kBinLen >> sub_shift consecutive sub-bins, contiguous in the buffer.
-  uint32_t *hist;           // [nsub][grid] counts, then offsets within the
-                            // sub-bin
-  uint32_t *tot;            // [nsub] events per sub-bin
-  uint32_t *bstart;         // [nb+1] first event of each bin
+  uint32_t *tot;            // [nb][kBinStride] events of each bin, in the
+                            // first element (0 between steps)
   uint32_t *cstart;         // [nb+1] first chunk of each bin
-  unsigned long long *ev;   // [ev_cap] (index within bin, value bits)
+  unsigned long long *ev;   // [nb][bin_cap] (index within bin, value bits)
   float *part;              // [chunk_cap][kBinLen] partial sums,
                             // chunk_cap = kReduceChunks + nb
-  uint32_t *meta;           // [2] chunk size of the step, and whether
-                            // some bin has more than one chunk
-  long long ev_cap;         // above this many events the step falls back
-                            // to atomic delivery
+  uint32_t *meta;           // [1] whether some bin has more than one chunk
+  uint32_t bin_cap;         // events beyond it in a bin are added with
+                            // float atomics
   int nb;                   // bins: ceil(acc_n / kBinLen)
-  int nsub;                 // sub-bins: ceil(acc_n >> sub_shift)
-  int sub_shift;
-  int grid;                 // blocks of the count and scatter phases
+  int grid;                 // blocks of the scatter
   long long acc_n;          // accumulator entries (ports x nodes)
 };
 
@@ -437,12 +431,16 @@ struct TileArgs {
 };
 constexpr float kTileHeightMax = 1024.0f;
 constexpr int kTiledPairTile = 32;  // most pairs per wave tile, tiled mode
+// LDS of a tiled block beside the tile and the pair prefix: the waves'
+// pair tables
+constexpr int kTiledScratch = kTiledBlock / 64 * 768;
 
 struct RevArgs {
   const uint32_t *ring_src;
   long long cap;
   int R;
   long long gs;
+  int slot;                           // gs % R
   const uint32_t *ring_n;
   const int *den_idx;
   int max_den;
@@ -496,7 +494,7 @@ const char *LaunchPoint(const PointArgs &a, void *stream);
 void LaunchExt(const ExtArgs &a, void *stream);
 void LaunchDelivery(const DeliveryArgs &a, int grid, void *stream);
 void LaunchClockSet(StepClock *c, const StepClock &v, void *stream);
-// Binned delivery: count, scan, scatter, reduce, sum (five launches).
+// Binned delivery: scatter, reduce, sum (three launches).
 // Requires a non-plastic network and b.nb <= kMaxBins.
 void LaunchDeliveryTiled(const DeliveryArgs &a, const TileArgs &b,
                          void *stream);
