@@ -64,6 +64,13 @@ inline int Rk5KindOf(int m) {
   }
 }
 
+// parameter row that the model's kernels write (refractory_step), or -1
+inline int RefractoryParam(int m) {
+  if (IsAeifCond(m)) return 12;
+  if (Rk5KindOf(m) >= 0) return m == kIzhikevichCondBeta ? 7 : 12;
+  return -1;
+}
+
 // the fixed-step models of point_models.hip: their PointKind, or -1
 inline int PointKindOf(int m) {
   switch (m) {
@@ -453,10 +460,12 @@ class Engine {
   void EnsureHostCSR();
   void BuildDeviceStore();
   // the rows of sources s0 .. s0+n-1 in three copies: base[0..n] (offsets
-  // into rec, relative to base[0]), seg[(D+1)*i ..] and rec
+  // into rec, relative to base[0]), seg[(D+1)*i ..] and rec; with sg also
+  // their synapse groups (empty in a network without plastic synapses)
   void SourceRangeRows(int s0, int n, std::vector<unsigned long long> &base,
                        std::vector<uint32_t> &seg,
-                       std::vector<unsigned long long> &rec);
+                       std::vector<unsigned long long> &rec,
+                       std::vector<uint8_t> *sg = nullptr);
   FoldIn MakeFold(long long pois_T, double pois_t);
   SpikeOut MakeSpikeOut(Group &g, long long T, double t);
 };
