@@ -1,6 +1,7 @@
-// Node update of the other RK5 neuron models: one neuron per lane, the
-// whole time step in one launch (adaptive Cash-Karp substeps with the
-// model's ExternalUpdate after each, as RK5Update does).
+// Node update of the other RK5 neuron models: the whole time step in one
+// launch (adaptive Cash-Karp substeps with the model's ExternalUpdate after
+// each, as RK5Update does), one neuron per lane, then a wave's last neurons
+// on quads of lanes.
 //
 //   aeif_psc_alpha  src/aeif_psc_alpha_kernel.h:132-201, aeif_psc_alpha.cu:24-68
 //   aeif_psc_exp    src/aeif_psc_exp_kernel.h:126-193, aeif_psc_exp.cu:24-62
@@ -19,6 +20,7 @@
 
 #include "ngpu_device.h"
 #include "ngpu_kernels.h"
+#include "rk5_quads.h"
 #include "step_common.h"
 
 namespace ngpu {
@@ -182,70 +184,224 @@ struct IzhModel {
   __device__ __forceinline__ float tref() const { return t_ref; }
 };
 
+// Derivatives of a current-based AdEx neuron on a quad of lanes (rk5_quads.h):
+// lane 0 V and w, lane 1 + p the currents of port p.
+template <int K, int P>
+struct PscQuad {
+  float V_th, Delta_T, inv_Delta_T, g_L, E_L, I_e, V_peak, V_reset;
+  float a;          // 0 in the port lanes
+  float ca, cb;     // 1/C_m and 1/tau_w, or 1/tau_syn twice
+  float V_b, n_refr;
+  float ca_now;     // ca, 0 for a refractory membrane
+  bool port, clamp;
+
+  __device__ __forceinline__ PscQuad(const PscModel<K, P> &m, float dt,
+                                     int role, int rv) {
+    V_th = m.V_th;
+    Delta_T = m.Delta_T;
+    inv_Delta_T = m.inv_Delta_T;
+    g_L = m.g_L;
+    E_L = m.E_L;
+    I_e = m.I_e;
+    V_peak = m.V_peak;
+    V_reset = m.V_reset;
+    port = role != 0;
+    a = role == 0 ? m.a : 0.0f;
+    ca = m.inv_C_m;
+    cb = m.inv_tau_w;
+#pragma unroll
+    for (int k = 0; k < P; k++)
+      if (rv == k + 1) ca = cb = m.inv_tau_syn[k];
+    V_b = m.b;
+    const int ri = (int)roundf(m.t_ref / dt);
+    n_refr = (float)(ri < 0 ? 0 : ri);
+  }
+  __device__ __forceinline__ void refractory(bool rf) {
+    clamp = port || rf;
+    ca_now = !port && rf ? 0.0f : ca;
+  }
+  __device__ __forceinline__ void rhs(float ya, float yb, float &da,
+                                      float &db) const {
+    float V;   // (a NaN gives V_peak, as y < V_peak ? y : V_peak does)
+    asm("v_min_f32 %0, %1, %2" : "=v"(V) : "v"(ya), "v"(V_peak));
+    V = clamp ? V_reset : V;
+    float I_syn = quad_get<1>(ya);
+    if constexpr (P > 1) I_syn = I_syn + quad_get<2>(ya);
+    if constexpr (P > 2) I_syn = I_syn + quad_get<3>(ya);
+    const float V_spike =
+        Delta_T == 0.0f ? 0.0f
+                        : Delta_T * dev_expf((V - V_th) * inv_Delta_T);
+    float t = (V - E_L) - V_spike;
+    t = (-g_L) * t;
+    t = t + I_syn;
+    t = t - yb;
+    t = t + I_e;
+    da = __builtin_fmaf(port ? -ya : t, ca_now, port ? yb : -0.0f);
+    float u = a * (V - E_L);
+    u = u - yb;
+    db = u * cb;
+  }
+};
+
+// One RK5 attempt of the lane's neuron with the step-boundary logic of
+// RK5Update and ExternalUpdate; true at the end of the time step.
+template <class M>
+__device__ __forceinline__ bool model_attempt(
+    const M &m, const Rk5ModelArgs &A, double x1, float (&y)[M::N],
+    const float (&k1)[M::N], const float (&scal)[M::N], double &x, float &h,
+    float &refr, int &nsp, int &n_att, bool &need_k1, int &n_acc,
+    int &n_rej) {
+  float yn[M::N];
+  const float h_max = (float)(x1 - x);
+  float hh = h;
+  if (hh > h_max) hh = h_max;
+  if (hh < A.h_min) hh = A.h_min;
+  const float err = rk5_attempt(m, refr, y, k1, scal, hh, A.eps, yn);
+  n_att++;
+  const bool accept = err <= 1.0f || (double)hh <= A.h_min_acc;
+  const float pw = dev_pow_ctrl(err, accept ? -0.2f : -0.25f);
+  const float hc = (hh * CK::coeff) * pw;
+  if (accept) {
+    n_acc++;
+    if (err > 1.0f) count_forced(A.forced);
+    x += (double)hh;
+    h = err > CK::err_min ? hc : 5.0f * hh;
+#pragma unroll
+    for (int k = 0; k < M::N; k++) y[k] = yn[k];
+  } else {
+    n_rej++;
+    if (n_att <= kMaxAttemptsPerStep) {
+      const float h_lo = 0.1f * hh;
+      h = hc > h_lo ? hc : h_lo;
+      return false;   // retry with the smaller step
+    }
+    h = hh;
+    x = x1;           // give up on this step
+  }
+  const bool end = x >= x1 - (double)A.h_min;
+  need_k1 = true;
+  if (y[0] < -1.0e3f || y[1] < -1.0e6f || y[1] > 1.0e6f) {
+    y[0] = m.reset_V();
+    y[1] = 0.0f;
+  } else if (refr > 0.0f) {
+    y[0] = m.reset_V();
+    if (end) refr -= 1.0f;
+  } else if (y[0] >= m.thresh()) {
+    nsp++;
+    y[0] = m.reset_V();
+    y[1] = y[1] + m.jump();
+    const int ri = (int)roundf(m.tref() / A.dt);
+    refr = (float)(ri < 0 ? 0 : ri);
+  }
+  return end;
+}
+
+// Models with a quad form (its type), for up to kQuadMaxPort ports.
+template <class M, int P>
+struct QuadOf {
+  static constexpr bool has = false;
+};
+template <int K, int P>
+struct QuadOf<PscModel<K, P>, P> {
+  static constexpr bool has = K != kRk5PscDelta && P <= kQuadMaxPort;
+  static constexpr int VP = K == kRk5PscAlpha ? 2 : 1;
+  using type = PscQuad<K, P>;
+};
+
+// One neuron per lane; every turn of the loop is one attempt of every
+// running neuron of the wave, whether it starts an RK5 step or retries one.
+// When at most 16 neurons of the wave are left they move to quads.
 template <class M, int P>
 __global__ __launch_bounds__(kBlock) void rk5_model_kernel(Rk5ModelArgs A) {
   constexpr int N = M::N;
   const StepNow sn = step_now(A.out, &A.fold, A.clock);
   const double x1 = A.clock ? sn.t : A.x1;
   int i = blockIdx.x * kBlock + threadIdx.x;
-  bool active = i < A.n;
-  int ii = active ? i : 0;
-  int node = A.i0 + ii;
+  const bool active = i < A.n;
+  if (!active) i = 0;
   int nsp = 0, n_acc = 0, n_rej = 0;
-  if (active) {
-    M m;
-    m.load(A.param, A.n, i);
-    float y[N];
+  M m;
+  m.load(A.param, A.n, i);
+  float y[N], k1[N], scal[N];
 #pragma unroll
-    for (int k = 0; k < N; k++) y[k] = A.var[(size_t)k * A.n + i];
+  for (int k = 0; k < N; k++) {
+    y[k] = A.var[(size_t)k * A.n + i];
+    scal[k] = 1.0f;
+  }
+  if (active) {
     float in[P];
-    gather_input<P>(A.fold, sn, node, in);
+    gather_input<P>(A.fold, sn, A.i0 + i, in);
     m.fold(y, in);
-    if (A.do_step) {
-      float *refr_p = A.param + (size_t)M::kRefrParam * A.n + i;
-      double x = A.x[i];
-      float h = A.h[i];
-      float refr = *refr_p;
-      int n_att = 0;
-      bool end = false;
-      while (!end) {
-        float hmax = (float)(x1 - x);
-        if (!rk5_step(m, refr, x, y, h, A.h_min, A.h_min_acc, hmax, A.eps,
-                      n_att, n_acc, n_rej, A.forced))
-          x = x1;
-        end = (x >= x1 - (double)A.h_min);
-        // ExternalUpdate
-        if (y[0] < -1.0e3f) {
-          y[0] = m.reset_V();
-          y[1] = 0.0f;
-          continue;
-        }
-        if (y[1] < -1.0e6f || y[1] > 1.0e6f) {
-          y[0] = m.reset_V();
-          y[1] = 0.0f;
-          continue;
-        }
-        if (refr > 0.0f) {
-          y[0] = m.reset_V();
-          if (end) refr -= 1.0f;
-        } else if (y[0] >= m.thresh()) {
-          nsp++;
-          y[0] = m.reset_V();
-          y[1] = y[1] + m.jump();
-          float r = roundf(m.tref() / A.dt);
-          int ri = (int)r;
-          refr = (float)(ri < 0 ? 0 : ri);
-        }
-      }
-      A.x[i] = x;
-      A.h[i] = h;
-      *refr_p = refr;
-    }
+  }
+  auto store = [&](float *refr_p, double x, float h, float refr) {
+    A.x[i] = x;
+    A.h[i] = h;
+    *refr_p = refr;
+  };
+  auto store_y = [&]() {
 #pragma unroll
     for (int k = 0; k < N; k++) A.var[(size_t)k * A.n + i] = y[k];
+  };
+  if (!A.do_step) {
+    if (active) store_y();
+    return;
   }
-  if (!A.do_step) return;
-  emit_spikes(A.out, sn, active, ii, node, nsp, (float)nsp);
+  float *refr_p = A.param + (size_t)M::kRefrParam * A.n + i;
+  double x = A.x[i];
+  float h = A.h[i];
+  float refr = *refr_p;
+  int n_att = 0;
+  bool run = active, need_k1 = true;
+  for (;;) {
+    const unsigned long long running = lanes_where(run);
+    if (running == 0ull) break;
+    if constexpr (QuadOf<M, P>::has) {
+      if (__popcll(running) <= kQuadsPerWave) {
+        constexpr int VP = QuadOf<M, P>::VP;
+        QuadState<P, VP> st;
+        st.take(run, i, y, scal, x, h, refr, nsp, n_att, need_k1);
+        M mq;
+        mq.load(A.param, A.n, st.i);
+        typename QuadOf<M, P>::type q(mq, A.dt, st.role, st.rv);
+        const QuadStep step = {x1, A.h_min, A.h_min_acc, A.eps, A.forced};
+        quad_run(
+            q, st, step, n_acc, n_rej,
+            [&](const QuadState<P, VP> &s, bool done) {
+              if (done && s.own) {
+                if (s.role == 0) {
+                  A.x[s.i] = s.x;
+                  A.h[s.i] = s.h;
+                  A.param[(size_t)M::kRefrParam * A.n + s.i] = s.refr;
+                }
+                const int k =
+                    s.role == 0 ? 0 : 2 + VP * (s.role - 1);
+                A.var[(size_t)k * A.n + s.i] = s.ya;
+                if (VP == 2 || s.role == 0)
+                  A.var[(size_t)(k + 1) * A.n + s.i] = s.yb;
+              }
+              const bool sp = done && s.role == 0;
+              emit_spikes(A.out, sn, sp, sp ? s.i : 0,
+                          A.i0 + (sp ? s.i : 0), s.nsp, (float)s.nsp);
+            });
+        break;
+      }
+    }
+    bool done = false;
+    if (run) {
+      if (need_k1) {
+        rk5_begin(m, refr, y, h, k1, scal);
+        need_k1 = false;
+      }
+      done = model_attempt(m, A, x1, y, k1, scal, x, h, refr, nsp, n_att,
+                           need_k1, n_acc, n_rej);
+      if (done) {
+        store(refr_p, x, h, refr);
+        store_y();
+        run = false;
+      }
+    }
+    emit_spikes(A.out, sn, done, i, A.i0 + i, nsp, (float)nsp);
+  }
   rk5_count(A.cnt, n_acc, n_rej);
 }
 

@@ -1,10 +1,13 @@
-"""The second RK5 pass's lane layouts: neurons on lanes of their own, then
-one neuron per quad of lanes for a wave's last neurons, against the
-single-pass kernel (one neuron a lane to the end of the step), bit for bit.
+"""The RK5 updates' lane layouts: neurons on lanes of their own, then one
+neuron per quad of lanes for a wave's last neurons.  The second pass of the
+AdEx conductance models against the single-pass kernel (one neuron a lane to
+the end of the step), the current-based models against the FP32 oracle, bit
+for bit.
 """
 import numpy as np
 import pytest
 
+import netbuild as nb
 from neurongpu_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +68,41 @@ def test_second_pass_layouts(ngpu, ports, uniform):
             assert np.array_equal(a, b)
         # the same attempts, accepted and rejected
         assert got[5] == want[5]
+
+
+@pytest.mark.parametrize("n", [1, 70, 300])
+@pytest.mark.parametrize("ports", [1, 2, 3, 4])
+@pytest.mark.parametrize("model", ["aeif_psc_alpha", "aeif_psc_exp"])
+def test_psc_layouts(ngpu, model, ports, n):
+    """1 neuron (quads from the start), a whole wave and some lanes, several
+    blocks; 4 ports keep one lane per neuron.  Delta_T = 0 in the largest."""
+    print("case psc_layouts", model, ports, n, flush=True)
+    rng = np.random.default_rng(100 * ports + n)
+    m = 10 * n
+    conns = [{"src": rng.integers(0, n, m), "tgt": rng.integers(0, n, m),
+              "weight": 8.0 * rng.integers(-2, 5, m),
+              "delay": 0.1 * rng.integers(1, 8, m), "port": q}
+             for q in range(ports)]
+    params = {"I_e": rng.uniform(700.0, 1500.0, n), "t_ref": 0.5,
+              "V_peak": 0.0, "tau_syn": [2.0, 1.0, 5.0, 3.0][:ports]}
+    if n == 300:
+        params["Delta_T"] = np.where(np.arange(n) % 5 == 0, 0.0, 2.0)
+    sp = {"seed": 7, "conns": conns, "groups": [
+        {"model": model, "n": n, "n_port": ports, "params": params,
+         "vars": {"V_m": rng.uniform(-70.0, -50.0, n).astype(np.float32)}}],
+        "records": [(i, v, 0) for i in (0, n // 2, n - 1)
+                    for v in ("V_m", "w")]}
+    groups, recs = nb.build_engine(ngpu, sp)
+    ngpu.ActivateSpikeCount(groups[0])
+    ngpu.Simulate(50.0)
+    net, _ = nb.build_oracle(sp, "f32")
+    net.run(500)
+    orc = net.records()
+    for k, r in enumerate(recs):
+        data = ngpu.GetRecordDataArray(r)
+        assert np.array_equal(orc[:, 1 + k].astype(np.float32), data[:, 1])
+    count = np.array(ngpu.GetNeuronIntVar(0, n, "spike_count"))
+    _, node, times = net.spikes()
+    want = np.zeros(n, int)
+    np.add.at(want, np.asarray(node, int), np.asarray(times, int))
+    assert np.array_equal(count, want) and count.sum() > 0
