@@ -270,6 +270,20 @@ class Engine {
   };
   std::vector<DeferredPass2> deferred_pass2;
   bool fuse_delivery = true;  // delivery in the last second-pass launch
+  // small networks: each AdEx group's step in one launch, the delivery with
+  // the last launch of an AdEx or iaf_psc_exp group (OneLaunchPays); the
+  // groups left for that
+  bool one_launch = false;
+  std::vector<DeferredPass2> deferred_step;
+  std::vector<IafArgs> deferred_iaf;
+  bool OneLaunchPays() const;
+  // accumulators: one-launch steps alternate between two sets, so that the
+  // delivery adds for the next step while the group reads its own; acc_set
+  // is the one the next fold reads
+  int acc_set = 0;
+  float *Acc(int other = 0) const {
+    return d_acc.p + (size_t)(acc_set ^ other) * (size_t)max_port * n_node;
+  }
   // learned RK5 step-size proposer
   DBuf<float> d_prop_w, d_prop_m, d_prop_v, d_prop_grad, d_prop_loss;
   DBuf<uint16_t> d_prop_bf16;

@@ -601,7 +601,10 @@ void aeif_pass1_kernel(AeifArgs A) {
     }
   }
   emit_spikes(A.out, sn, active && finished, ii, node, nsp, (float)nsp);
-  rk5_count(A.cnt1 ? A.cnt1 : A.cnt, n_acc, n_rej);
+  if (B1)
+    rk5_count_one(A.cnt1 ? A.cnt1 : A.cnt, n_acc, n_rej);
+  else
+    rk5_count(A.cnt1 ? A.cnt1 : A.cnt, n_acc, n_rej);
   if (OV && A.mask_write) {
     const unsigned long long m =
         __ballot(slot != 0xFFFFFFFFu || cslot != 0xFFFFFFFFu);
@@ -1034,12 +1037,99 @@ void aeif_tail_kernel(AeifArgs A, DeliveryArgs D, uint32_t n2) {
     delivery_body<false>(clocked(D), blockIdx.x - n2, gridDim.x - n2);
 }
 
+// Whole time step of a group of at most kOneLaunchMax neurons: every attempt
+// of its neurons, the last ones of a wave on quads of lanes.
+template <int P, bool UNI>
+__device__ __forceinline__ void aeif_step_body(const AeifArgs &A,
+                                               uint32_t vblock) {
+  constexpr int N = 2 + 2 * P;
+  const StepNow sn = step_now(A.out, &A.fold, A.clock);
+  const double x1 = A.clock ? sn.t : A.x1;
+  // (the two-pass update finds the next step's list lengths cleared)
+  if (vblock == 0 && threadIdx.x < 2 * kStragLists)
+    A.strag_n2[2 * kStragLists * ((aeif_gs(A) + 1) & 3) + threadIdx.x] = 0u;
+  int i = vblock * kBlock + threadIdx.x;
+  const bool active = i < A.n;
+  if (!active) i = 0;
+  AeifLocal<P> p;
+  aeif_load_params<P, UNI>(A, i, p);
+  float y[N], k1[N], scal[N];
+  const uint32_t u = (uint32_t)i;
+  y[0] = at(A.V, u);
+  y[1] = at(A.w, u);
+#pragma unroll
+  for (int q = 0; q < P; q++) {
+    y[2 + 2 * q] = at(A.g[q], u);
+    y[3 + 2 * q] = at(A.g1[q], u);
+  }
+  double x = at(A.x, u);
+  float h = at(A.h, u);
+  float refr = at(A.refr, u);
+  if (active) {
+    float in[P];
+    gather_input<P>(A.fold, sn, A.i0 + i, in);
+#pragma unroll
+    for (int q = 0; q < P; q++)
+      y[3 + 2 * q] = __builtin_fmaf(in[q], p.g0[q], y[3 + 2 * q]);
+  }
+  int nsp = 0, n_att = 0, n_acc = 0, n_rej = 0;
+  bool need_k1 = true, run = active, first = true;
+  float err = 1.0f, hh = 0.0f;
+  for (;;) {
+    const unsigned long long running = lanes_where(run);
+    if (running == 0ull) break;
+    if (!first && __popcll(running) <= kQuadsPerWave) {
+      aeif_quad_finish<P, UNI>(late_args(), sn, x1, run, i, y, scal, x, h,
+                               refr, nsp, n_att, need_k1, n_acc, n_rej);
+      break;
+    }
+    bool done = false;
+    if (run) {
+      if (need_k1) {
+        aeif_rk5_begin<P>(p, refr, y, h, k1, scal);
+        need_k1 = false;
+      }
+      done = aeif_attempt_and_update<P>(A, x1, p, y, k1, scal, x, h, refr,
+                                        nsp, n_att, need_k1, n_acc, n_rej,
+                                        err, hh);
+      if (done) {
+        aeif_store_state<P>(A, i, y, x, h, refr);
+        run = false;
+      }
+    }
+    emit_spikes(A.out, sn, done, i, A.i0 + i, nsp, (float)nsp);
+    if (first) {
+      rk5_count_one(A.cnt1 ? A.cnt1 : A.cnt, n_acc, n_rej);
+      n_acc = n_rej = 0;
+      first = false;
+    }
+  }
+  aeif_count<P>(A, n_acc, n_rej);
+}
+
+// The whole step of a small network in one launch: blocks [0, n1) the group,
+// the others the step's atomic delivery, which reads earlier steps' spikes
+// and adds to the accumulators that the next step reads (D.acc, not the ones
+// that this step's fold reads).  A step of 1000 quiet neurons is two
+// dependent launches of 6.6 and 2.8 us otherwise (first pass; empty second
+// pass and delivery), and with spiking neurons the chain of the slowest one
+// waits for every first attempt.
+template <int P, bool UNI>
+__global__ __launch_bounds__(kBlock) void aeif_step_kernel(AeifArgs A,
+                                                           DeliveryArgs D,
+                                                           uint32_t n1) {
+  if (blockIdx.x < n1)
+    aeif_step_body<P, UNI>(A, blockIdx.x);
+  else
+    delivery_body<false>(D, blockIdx.x - n1, gridDim.x - n1);
+}
+
 // ---------------------------------------------------------------------
 // iaf_psc_exp, exact integration (src/iaf_psc_exp.cu:94-119)
 // ---------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void iaf_kernel(IafArgs A) {
+__device__ __forceinline__ void iaf_body(const IafArgs &A, uint32_t vblock) {
   const StepNow sn = step_now(A.out, &A.fold, A.clock);
-  int i = blockIdx.x * kBlock + threadIdx.x;
+  int i = vblock * kBlock + threadIdx.x;
   bool active = i < A.n;
   int ii = active ? i : 0;
   int node = A.i0 + ii;
@@ -1076,6 +1166,21 @@ __global__ __launch_bounds__(kBlock) void iaf_kernel(IafArgs A) {
   }
   if (!A.do_step) return;
   emit_spikes(A.out, sn, active, ii, node, nsp, 1.0f);
+}
+
+__global__ __launch_bounds__(kBlock) void iaf_kernel(IafArgs A) {
+  iaf_body(A, blockIdx.x);
+}
+
+// Small networks: the update and the step's atomic delivery in one launch,
+// as aeif_step_kernel.
+__global__ __launch_bounds__(kBlock) void iaf_step_kernel(IafArgs A,
+                                                          DeliveryArgs D,
+                                                          uint32_t n1) {
+  if (blockIdx.x < n1)
+    iaf_body(A, blockIdx.x);
+  else
+    delivery_body<false>(D, blockIdx.x - n1, gridDim.x - n1);
 }
 
 // ---------------------------------------------------------------------
@@ -2361,6 +2466,32 @@ void LaunchAeifPass2(const AeifArgs &a, int n_port, const DeliveryArgs *d,
   }
 }
 
+void LaunchAeifStep(const AeifArgs &a, int n_port, const DeliveryArgs *d,
+                    int d_grid, void *stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const uint32_t n1 = (uint32_t)((a.n + kBlock - 1) / kBlock);
+  const DeliveryArgs da = d ? *d : DeliveryArgs{};
+  const dim3 grid(n1 + (d ? (uint32_t)d_grid : 0u));
+  const size_t lds = d ? delivery_lds_bytes(d->D, 0) : 0;
+  if (n1 == 0) return;
+#define NGPU_STEP(P)                                                        \
+  case P:                                                                   \
+    if (a.uniform)                                                          \
+      hipLaunchKernelGGL((aeif_step_kernel<P, true>), grid, dim3(kBlock),   \
+                         lds, s, a, da, n1);                                \
+    else                                                                    \
+      hipLaunchKernelGGL((aeif_step_kernel<P, false>), grid, dim3(kBlock),  \
+                         lds, s, a, da, n1);                                \
+    break;
+  switch (n_port) {
+    NGPU_STEP(1)
+    NGPU_STEP(2)
+    NGPU_STEP(3)
+    default: break;
+  }
+#undef NGPU_STEP
+}
+
 void LaunchAeif(const AeifArgs &a, int n_port, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   switch (n_port) {
@@ -2380,6 +2511,14 @@ void LaunchIaf(const IafArgs &a, void *stream) {
   if (grid > 0)
     hipLaunchKernelGGL(iaf_kernel, dim3(grid), dim3(kBlock), 0,
                        (hipStream_t)stream, a);
+}
+
+void LaunchIafStep(const IafArgs &a, const DeliveryArgs &d, int d_grid,
+                   void *stream) {
+  const uint32_t n1 = (uint32_t)((a.n + kBlock - 1) / kBlock);
+  hipLaunchKernelGGL(iaf_step_kernel, dim3(n1 + (uint32_t)d_grid),
+                     dim3(kBlock), delivery_lds_bytes(d.D, 0),
+                     (hipStream_t)stream, a, d, n1);
 }
 
 void LaunchRelay(const RelayArgs &a, void *stream) {

@@ -484,7 +484,15 @@ const char *PropEvalNoAlloc(const unsigned char *pk, const float *feat,
 // the step (non-plastic) runs in the same launch on d_grid more blocks
 void LaunchAeifPass2(const AeifArgs &a, int n_port, const DeliveryArgs *d,
                      int d_grid, void *stream);
+// whole step of a small group in one launch, with d != nullptr the atomic
+// delivery on d_grid more blocks; up to kOneLaunchPorts ports
+constexpr int kOneLaunchMax = 65536;   // neurons: one wave per SIMD
+constexpr int kOneLaunchPorts = 3;
+void LaunchAeifStep(const AeifArgs &a, int n_port, const DeliveryArgs *d,
+                    int d_grid, void *stream);
 void LaunchIaf(const IafArgs &a, void *stream);
+void LaunchIafStep(const IafArgs &a, const DeliveryArgs &d, int d_grid,
+                   void *stream);
 // returns an error message, or nullptr
 const char *LaunchRk5Model(const Rk5ModelArgs &a, void *stream);
 void LaunchRelay(const RelayArgs &a, void *stream);

@@ -367,5 +367,18 @@ __device__ __forceinline__ void rk5_count(unsigned long long *cnt, int n_acc,
   }
 }
 
+// The same for at most one attempt per lane: two ballots instead of two
+// cross-lane sums.
+__device__ __forceinline__ void rk5_count_one(unsigned long long *cnt,
+                                              int n_acc, int n_rej) {
+  const int sa = (int)__popcll(__ballot(n_acc > 0));
+  const int sr = (int)__popcll(__ballot(n_rej > 0));
+  if (lane_id() == 0 && cnt && (sa | sr)) {
+    unsigned long long *c = cnt + 2 * (blockIdx.x & (kCounterSlots - 1));
+    if (sa) atomicAdd(c, (unsigned long long)sa);
+    if (sr) atomicAdd(c + 1, (unsigned long long)sr);
+  }
+}
+
 }  // namespace
 }  // namespace ngpu

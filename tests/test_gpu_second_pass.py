@@ -106,3 +106,57 @@ def test_psc_layouts(ngpu, model, ports, n):
     want = np.zeros(n, int)
     np.add.at(want, np.asarray(node, int), np.asarray(times, int))
     assert np.array_equal(count, want) and count.sum() > 0
+
+
+def test_switches_between_step_forms(ngpu):
+    """Two AdEx groups and an iaf_psc_exp group coupled by dyadic synapses:
+    steps in one launch, in two passes and binned with overlap, switched
+    between and within Simulate calls, against single-pass steps."""
+    print("case step_forms", flush=True)
+    rng = np.random.default_rng(17)
+    n = [300, 200, 150]
+    off = [0, 300, 500]
+    conns = []
+    for s in range(3):
+        for t in range(3):
+            m = 4000
+            conns.append({"src": off[s] + rng.integers(0, n[s], m),
+                          "tgt": off[t] + rng.integers(0, n[t], m),
+                          "weight": 0.25 if t < 2 else 16.0,
+                          "delay": 0.1 * rng.integers(1, 12, m), "port": 0})
+    sp = {"seed": 5, "conns": conns, "groups": [
+        {"model": "aeif_cond_beta", "n": n[0], "n_port": 2,
+         "params": {"I_e": 800.0, "t_ref": 0.3},
+         "vars": {"V_m": rng.uniform(-70., -40., n[0]).astype(np.float32)}},
+        {"model": "aeif_cond_alpha", "n": n[1], "n_port": 1,
+         "params": {"I_e": rng.uniform(600.0, 900.0, n[1])}},
+        {"model": "iaf_psc_exp", "n": n[2], "params": {"I_e": 500.0}}]}
+
+    def go(phases):
+        groups, _ = wl.build_from_spec(ngpu, sp)
+        for g in groups:
+            ngpu.ActivateSpikeCount(g)
+        out = []
+        for st in phases:
+            ngpu.SetKernelStatus(st)
+            ngpu.SetSimTime(7.0)
+            ngpu.StartSimulation()
+            for k in range(70):
+                if k == 35 and st.get("delivery_mode") == 1:
+                    ngpu.SetKernelStatus("delivery_mode", 0)
+                ngpu.SimulationStep()
+            ngpu.EndSimulation()
+            out += [np.array(ngpu.GetNeuronVar(g.i0, g.n, v)) for g, v in
+                    zip(groups, ("V_m", "g1", "V_m_rel"))]
+            out += [np.array(ngpu.GetNeuronIntVar(g.i0, g.n, "spike_count"))
+                    for g in groups]
+        return out
+
+    one = {"rk5_two_pass": 1, "fuse_delivery": 1, "delivery_mode": 0}
+    two = dict(one, fuse_delivery=0)
+    bins = dict(one, delivery_mode=1)
+    want = go([dict(one, rk5_two_pass=0)] * 7)
+    got = go([one, two, one, bins, one, bins, two])
+    assert want[-1].sum() > 0 and want[-3].sum() > 0
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
