@@ -27,7 +27,9 @@ const char *BuildReverseIndex(const unsigned long long *rec,
 
 // Tile-major copy of the canonical store for the tiled delivery: trec
 // (S records) holds the records grouped by accumulator tile
-// ((port * n_total + target) >> tile_shift), canonical order inside a tile;
+// ((port * n_total + target) >> tile_shift), canonical order inside a tile,
+// with the entry within the tile in the low word instead of the target and
+// port (the delivery then needs no quarter-rate product per event);
 // off ((N*D + 1) * T entries) gets off[(s*D + d)*T + t] = position in trec
 // of the first record of source s, delay slot d in tile t (row N*D: the
 // tile ends).  Requires S < 2^31 and T*N*D < 2^31.  Returns null on

@@ -139,8 +139,8 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t m) {
 constexpr int kBoundBlock = 1024;
 __global__ __launch_bounds__(kBoundBlock) void tile_bound(
     const unsigned long long *trec, const uint32_t *off, unsigned long long nd,
-    uint32_t T, int tile_shift, long long n_total, uint32_t gb,
-    uint32_t *bound, uint32_t *wmax) {
+    uint32_t T, int tile_shift, uint32_t gb, uint32_t *bound,
+    uint32_t *wmax) {
   extern __shared__ uint32_t s_cnt[];
   __shared__ uint32_t s_red[2];
   const uint32_t t = blockIdx.x / gb, k = blockIdx.x - t * gb;
@@ -151,14 +151,10 @@ __global__ __launch_bounds__(kBoundBlock) void tile_bound(
   const uint32_t r0 = off[t], n = off[nd * T + t] - r0;
   const uint32_t c0 = r0 + (uint32_t)((unsigned long long)n * k / gb);
   const uint32_t c1 = r0 + (uint32_t)((unsigned long long)n * (k + 1) / gb);
-  const long long a0 = (long long)t << tile_shift;
   uint32_t wb = 0;
   for (uint32_t j = c0 + threadIdx.x; j < c1; j += kBoundBlock) {
     const unsigned long long r = trec[j];
-    const uint32_t tp = (uint32_t)r;
-    const long long a =
-        (long long)(tp >> kPortShift) * n_total + (tp & kTargetMask);
-    atomicAdd(&s_cnt[a - a0], 1u);
+    atomicAdd(&s_cnt[(uint32_t)r], 1u);
     const uint32_t x = (uint32_t)(r >> 32) & 0x7FFFFFFFu;
     wb = x > wb ? x : wb;
   }
@@ -179,10 +175,19 @@ __global__ __launch_bounds__(kBoundBlock) void tile_bound(
   }
 }
 
-__global__ void gather_u64(const uint32_t *idx, const unsigned long long *src,
-                           unsigned long long S, unsigned long long *dst) {
+// Records of the tiled store: the entry within its tile in the low word
+// instead of the target and port.
+__global__ void gather_tiled(const uint32_t *idx, const unsigned long long *in,
+                             unsigned long long n, long long n_total,
+                             int tile_shift, unsigned long long *out) {
   unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < S) dst[i] = src[idx[i]];
+  if (i >= n) return;
+  const unsigned long long r = in[idx[i]];
+  const uint32_t tp = (uint32_t)r;
+  const unsigned long long a =
+      (unsigned long long)(tp >> kPortShift) * (unsigned long long)n_total +
+      (tp & kTargetMask);
+  out[i] = (r & 0xFFFFFFFF00000000ull) | (a & ((1ull << tile_shift) - 1ull));
 }
 
 // Records per (tile, source, delay slot), tile-major: one wavefront per
@@ -373,8 +378,8 @@ const char *BuildTiledStore(const unsigned long long *rec,
     if (hipcub::DeviceRadixSort::SortPairs(tmp.p, sort_bytes, kb, vb, (int)S,
                                            0, end_bit, stream) != hipSuccess)
       return "radix sort failed";
-    hipLaunchKernelGGL(gather_u64, dim3(grid), dim3(256), 0, stream,
-                       vb.Current(), rec, S, trec);
+    hipLaunchKernelGGL(gather_tiled, dim3(grid), dim3(256), 0, stream,
+                       vb.Current(), rec, S, n_total, tile_shift, trec);
     // the sort buffers are freed at the end of this scope
     if (hipStreamSynchronize(stream) != hipSuccess)
       return "tiled store build failed";
@@ -430,7 +435,7 @@ const char *TiledSumBound(const unsigned long long *trec, const uint32_t *off,
   }
   const uint32_t gb = 32;
   hipLaunchKernelGGL(tile_bound, dim3(T * gb), dim3(kBoundBlock), lds, stream,
-                     trec, off, nd, T, tile_shift, n_total, gb, tb.p,
+                     trec, off, nd, T, tile_shift, gb, tb.p,
                      tb.p + T);
   std::vector<uint32_t> h(T + 1);
   if (hipMemcpyAsync(h.data(), tb.p, (T + 1) * sizeof(uint32_t),

@@ -1127,6 +1127,8 @@ __global__ __launch_bounds__(kBlock) void aeif_step_kernel(AeifArgs A,
 // ---------------------------------------------------------------------
 // iaf_psc_exp, exact integration (src/iaf_psc_exp.cu:94-119)
 // ---------------------------------------------------------------------
+// (all threads of a block take part: the spikes leave with one atomic per
+// block)
 __device__ __forceinline__ void iaf_body(const IafArgs &A, uint32_t vblock) {
   const StepNow sn = step_now(A.out, &A.fold, A.clock);
   int i = vblock * kBlock + threadIdx.x;
@@ -1165,7 +1167,7 @@ __device__ __forceinline__ void iaf_body(const IafArgs &A, uint32_t vblock) {
     A.I_in[i] = I_in;
   }
   if (!A.do_step) return;
-  emit_spikes(A.out, sn, active, ii, node, nsp, 1.0f);
+  emit_spikes_block(A.out, sn, active, ii, node, nsp, 1.0f);
 }
 
 __global__ __launch_bounds__(kBlock) void iaf_kernel(IafArgs A) {
@@ -2117,20 +2119,19 @@ __global__ __launch_bounds__(kTiledBlock) void tiled_delivery_kernel(
   auto add = [&](bool ok, uint32_t, unsigned long long, unsigned long long r,
                  float hj, uint32_t) {
     if (!ok) return;
-    const uint32_t tp = (uint32_t)r;
-    const uint32_t idx = acc_index(tp, A.n_total);
+    const uint32_t loc = (uint32_t)r;   // entry of the tile
     const float v = hj * __uint_as_float((uint32_t)(r >> 32));
     if (FIXED) {
       if (fabsf(hj) <= B.h_max) {
         // exact: v * 2^F is v with a larger exponent, below 2^62
         const long long q = __float2ll_rn(v * B.q_scale);
-        atomicAdd(&s_q[idx - a0], (unsigned long long)q);
+        atomicAdd(&s_q[loc], (unsigned long long)q);
       } else {
-        unsafeAtomicAdd(A.acc + idx, v);
+        unsafeAtomicAdd(A.acc + a0 + loc, v);
         s_big = 1;
       }
     } else {
-      lds_add_f32(&s_acc[idx - a0], v);
+      lds_add_f32(&s_acc[loc], v);
     }
   };
   const unsigned long long n_events =

@@ -402,7 +402,8 @@ constexpr int kTileShiftMax = 15;
 constexpr int kTiledBlock = 1024;
 
 struct TileArgs {
-  const unsigned long long *trec;  // [S] tile-major records
+  const unsigned long long *trec;  // [S] tile-major records: entry within
+                                   // the tile, weight in the high word
   const uint32_t *off;             // [(N*D + 1) * T]: off[(s*D + d)*T + t]
                                    // = first record of (s, d) in tile t;
                                    // the next row ends it

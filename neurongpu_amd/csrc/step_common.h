@@ -58,22 +58,12 @@ __device__ __forceinline__ StepNow step_now(const SpikeOut &o, const FoldIn *f,
   return s;
 }
 
-// Wavefront-aggregated append of this lane's spikes to the ring slot of the
-// step, plus the per-node bookkeeping of PushSpike.
-__device__ __forceinline__ void emit_spikes(const SpikeOut &o,
-                                            const StepNow &sn, bool active,
-                                            int i, int node, int nsp,
-                                            float height) {
-  bool spk = active && nsp > 0;
-  unsigned long long mask = __ballot(spk);
-  if (mask == 0ull) return;
-  uint32_t leader = (uint32_t)(__ffsll((long long)mask) - 1);
-  uint32_t base = 0;
-  if (lane_id() == leader)
-    base = atomicAdd(sn.ring_n, (uint32_t)__popcll(mask));
-  base = __shfl(base, (int)leader);
-  if (!spk) return;
-  uint32_t pos = base + lanes_below(mask);
+// A spike at place pos of the ring slot, and the per-node bookkeeping of
+// PushSpike.
+__device__ __forceinline__ void put_spike(const SpikeOut &o,
+                                          const StepNow &sn, uint32_t pos,
+                                          int i, int node, int nsp,
+                                          float height) {
   sn.ring_src[pos] = (uint32_t)node;
   sn.ring_h[pos] = height;
   sn.ring_cnt[pos] = (uint32_t)nsp;
@@ -90,6 +80,52 @@ __device__ __forceinline__ void emit_spikes(const SpikeOut &o,
     }
     o.n_rec_times[i] = nr;
   }
+}
+
+// Wavefront-aggregated append of this lane's spikes to the ring slot of the
+// step.
+__device__ __forceinline__ void emit_spikes(const SpikeOut &o,
+                                            const StepNow &sn, bool active,
+                                            int i, int node, int nsp,
+                                            float height) {
+  bool spk = active && nsp > 0;
+  unsigned long long mask = __ballot(spk);
+  if (mask == 0ull) return;
+  uint32_t leader = (uint32_t)(__ffsll((long long)mask) - 1);
+  uint32_t base = 0;
+  if (lane_id() == leader)
+    base = atomicAdd(sn.ring_n, (uint32_t)__popcll(mask));
+  base = __shfl(base, (int)leader);
+  if (!spk) return;
+  put_spike(o, sn, base + lanes_below(mask), i, node, nsp, height);
+}
+
+// The same for a whole block, with one atomic for its spikes: where a large
+// part of the waves has spikes every step, an atomic per wave on the slot's
+// one counter is what the update waits for (77169 neurons at 434 Hz, 1200
+// waves: 15.6 us, 10.8 with one per block).  Every thread of the block calls it.
+__device__ __forceinline__ void emit_spikes_block(const SpikeOut &o,
+                                                  const StepNow &sn,
+                                                  bool active, int i,
+                                                  int node, int nsp,
+                                                  float height) {
+  __shared__ uint32_t s_first[kBlock / 64], s_base;
+  const bool spk = active && nsp > 0;
+  const unsigned long long mask = __ballot(spk);
+  const int wave = threadIdx.x / 64;
+  if (lane_id() == 0) s_first[wave] = (uint32_t)__popcll(mask);
+  __syncthreads();
+  uint32_t first = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; w++) {
+    first += w < wave ? s_first[w] : 0u;
+    all += s_first[w];
+  }
+  if (all == 0u) return;
+  if (threadIdx.x == 0) s_base = atomicAdd(sn.ring_n, all);
+  __syncthreads();
+  if (spk)
+    put_spike(o, sn, s_base + first + lanes_below(mask), i, node, nsp, height);
 }
 
 // Poisson count of a uniform draw u: the number of the table's
