@@ -804,7 +804,10 @@ __device__ __forceinline__ void aeif_pass2_body(const AeifArgs &A0,
                                                               : 64u;
   const uint32_t per_block = per_wave * (kBlock / 64);
   if (vblock * per_block >= total) return;  // whole block beyond the list
-  const AeifArgs &A = late_args();
+  // With the proposer every attempt runs in the lane loop below, where late
+  // arguments would be read again after each store: it takes them as passed
+  // (1e6 spiking neurons, tol 1e-6, 100 ms: 134 -> 132 ms in the mean).
+  const AeifArgs &A = PROP ? A0 : late_args();
   // the pass is a few long dependent chains: its waves issue first when
   // they share a SIMD with the first pass or the delivery
   if (CU) __builtin_amdgcn_s_setprio(3);
