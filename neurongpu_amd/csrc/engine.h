@@ -207,6 +207,7 @@ class Engine {
   bool rk5_two_pass = true;
   int rk5_budget = 1;          // RK5 attempts per neuron in the first pass
   int rk5_pass2_grid = 256;   // blocks of the second pass
+  void SetTwoPass(bool on);
   bool calibrated = false;
   bool first_simulation = true;
   bool in_simulation = false;

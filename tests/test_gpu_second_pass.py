@@ -160,3 +160,41 @@ def test_switches_between_step_forms(ngpu):
     assert want[-1].sum() > 0 and want[-3].sum() > 0
     for a, b in zip(want, got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("settings", [{"fuse_delivery": 0},
+                                      {"delivery_mode": 1}])
+@pytest.mark.parametrize("lengths", [(9, 1, 9), (10, 2, 8), (11, 3, 7),
+                                     (9, 36, 12)])
+def test_two_pass_switched_off_and_on(ngpu, settings, lengths):
+    """rk5_two_pass 1, 0, 1 between steps of one run, the single-pass steps
+    of every length modulo the four sets of lists, with second passes that
+    end their step and with overlapped ones: as in single-pass steps alone."""
+    print("case two_pass_switch", settings, lengths, flush=True)
+    sp = spec(2, True)
+
+    def go(passes):
+        groups, _ = wl.build_from_spec(ngpu, sp)
+        ngpu.SetKernelStatus(settings)
+        ngpu.ActivateSpikeCount(groups[0])
+        ngpu.SetSimTime(0.1 * sum(lengths) * 6)
+        ngpu.StartSimulation()
+        for _ in range(6):
+            for on, steps in zip(passes, lengths):
+                ngpu.SetKernelStatus("rk5_two_pass", on)
+                for _ in range(steps):
+                    ngpu.SimulationStep()
+        ngpu.EndSimulation()
+        out = [np.array(ngpu.GetNeuronVar(0, N, v))
+               for v in ("V_m", "w", "g", "g1")]
+        out.append(np.array(ngpu.GetNeuronIntVar(0, N, "spike_count")))
+        return out, ngpu.GetHotPathStats()
+
+    want, st_want = go((0, 0, 0))
+    got, st_got = go((1, 0, 1))
+    assert want[4].sum() > 0
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
+    assert st_got["syn_events"] == st_want["syn_events"]
+    assert st_got["rk5_accepted"] == st_want["rk5_accepted"]
+    assert st_got["rk5_rejected"] == st_want["rk5_rejected"]
