@@ -1524,48 +1524,76 @@ struct WaveTile {
     nz = __ballot(cnt > 0u);
   }
 
+  // Walked one pair at a time (walk), else spread over the wave (spread).
+  __device__ __forceinline__ bool long_segments() const {
+    return E > 64u * PairTable<WIDE>::kWords ||
+           E >= kLongSegment * (uint32_t)__popcll(nz);
+  }
+
   template <class F>
   __device__ __forceinline__ void emit(PairTable<WIDE> &tab,
                                        const unsigned long long *recs,
                                        F &&f) const {
     if (E == 0u) return;
+    if (long_segments())
+      walk<false>(recs, 0u, E, f);
+    else
+      spread(tab, recs, f);
+  }
+
+  // Events lo .. hi-1 of the tile (PART, else all), one pair at a time, its
+  // data broadcast through scalar registers, consecutive lanes on
+  // consecutive records.
+  template <bool PART, class F>
+  __device__ __forceinline__ void walk(const unsigned long long *recs,
+                                       uint32_t lo, uint32_t hi,
+                                       F &&f) const {
     const uint32_t lane = lane_id();
     const uint32_t pre = incl - cnt;
-    if (E > 64u * PairTable<WIDE>::kWords ||
-        E >= kLongSegment * (uint32_t)__popcll(nz)) {
-      // Long segments: one pair at a time, its data broadcast through
-      // scalar registers, consecutive lanes on consecutive records.
-      unsigned long long m = nz;
-      while (m) {
-        const int j = __ffsll((unsigned long long)m) - 1;
-        m &= m - 1ull;
-        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cnt, j);
-        const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)pre, j);
-        const uint32_t slo =
-            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)start, j);
-        const uint32_t shi =
-            (uint32_t)__builtin_amdgcn_readlane((int)(start >> 32), j);
-        const unsigned long long st = ((unsigned long long)shi << 32) | slo;
-        const float h = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(
-            (int)__float_as_uint(height), j));
-        const uint32_t mu = (uint32_t)__builtin_amdgcn_readlane((int)mult, j);
-        for (uint32_t o = 0; o < c; o += 64u * U) {
-          unsigned long long syn[U], r[U];
-          bool ok[U];
-#pragma unroll
-          for (int u = 0; u < U; u++) {
-            uint32_t e = o + 64u * u + lane;
-            ok[u] = e < c;
-            syn[u] = st + e;
-            r[u] = ok[u] ? recs[syn[u]] : 0ull;
-          }
-#pragma unroll
-          for (int u = 0; u < U; u++)
-            f(ok[u], pj + o + 64u * u + lane, syn[u], r[u], h, mu);
-        }
+    unsigned long long m = nz;
+    while (m) {
+      const int j = __ffsll((unsigned long long)m) - 1;
+      m &= m - 1ull;
+      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cnt, j);
+      const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)pre, j);
+      uint32_t o0 = 0u, o1 = c;
+      if (PART) {
+        if (pj + c <= lo) continue;
+        if (pj >= hi) break;
+        o0 = pj < lo ? lo - pj : 0u;
+        o1 = hi - pj < c ? hi - pj : c;
       }
-      return;
+      const uint32_t slo =
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)start, j);
+      const uint32_t shi =
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(start >> 32), j);
+      const unsigned long long st = ((unsigned long long)shi << 32) | slo;
+      const float h = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(
+          (int)__float_as_uint(height), j));
+      const uint32_t mu = (uint32_t)__builtin_amdgcn_readlane((int)mult, j);
+      for (uint32_t o = o0; o < o1; o += 64u * U) {
+        unsigned long long syn[U], r[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t e = o + 64u * u + lane;
+          ok[u] = e < o1;
+          syn[u] = st + e;
+          r[u] = ok[u] ? recs[syn[u]] : 0ull;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          f(ok[u], pj + o + 64u * u + lane, syn[u], r[u], h, mu);
+      }
     }
+  }
+
+  template <class F>
+  __device__ __forceinline__ void spread(PairTable<WIDE> &tab,
+                                         const unsigned long long *recs,
+                                         F &&f) const {
+    const uint32_t lane = lane_id();
+    const uint32_t pre = incl - cnt;
     // the tile's table (every lane has read the one before: its last group
     // was handed over)
     if (lane < (E + 63u) / 64u) tab.last[lane] = 0ull;
@@ -1746,6 +1774,9 @@ __global__ __launch_bounds__(kBlock) void delivery_kernel(DeliveryArgs A) {
 
 constexpr int kReduceBlock = 1024;
 constexpr int kBinBlock = 512;  // threads per block of the scatter
+// events of a tile of long segments that a wave buffers at a time: a
+// wave's share of the block's buffer
+constexpr uint32_t kBinPiece = kBinBuffer / (kBinBlock / 64);
 
 // Float add into LDS by compare-and-swap.  On gfx950 the LDS float atomic
 // add runs at about a twelfth of the rate of the integer atomics and of a
@@ -1832,12 +1863,19 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
   if (threadIdx.x == 0) s_n = 0u;
   const uint32_t total = delivery_prologue<kBinBlock>(
       A, blockIdx.x, s_pre, reinterpret_cast<uint32_t *>(s_tab));
-  const TileSplit<true> t = TileSplit<true>::make<kBinBlock>(
+  TileSplit<true> t = TileSplit<true>::make<kBinBlock>(
       total, (uint32_t)A.tile_max, blockIdx.x, gridDim.x);
+  // Tiles for at most half of the waves: spread over the blocks, whose
+  // buffers then take them side by side (50 pairs of 20000 events: 206 us
+  // per step in 7 blocks, 88 in 50).  More tiles stay in order, a block's
+  // next to each other in the ring (1e6 neurons: 0.9 % of a step).
+  if (t.n_tiles <= t.n_waves / 2u)
+    t.wave = threadIdx.x / 64 * gridDim.x + blockIdx.x;
   unsigned long long n_events = 0;
   uint32_t wt = t.wave;
   WaveTile<4, true> w;
   bool loaded = false;
+  uint32_t done = 0;                   // events of the tile in the buffer
   for (;;) {
     // round: every wave buffers its tiles until one does not fit
     bool waits = false;
@@ -1847,35 +1885,39 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
         n_events += w.E;
         loaded = true;
       }
-      if (w.E > (uint32_t)kBinBuffer) {
-        // more than any buffer holds: float atomics
-        w.emit(s_tab[threadIdx.x / 64], A.rec,
-               [&](bool ok, uint32_t, unsigned long long,
-                   unsigned long long r, float hj, uint32_t) {
-                 if (ok)
-                   unsafeAtomicAdd(A.acc + acc_index((uint32_t)r, A.n_total),
-                                   hj * __uint_as_float((uint32_t)(r >> 32)));
-               });
+      // Tiles of long segments go to the buffer in pieces, so that their
+      // size is not limited and the waves of a block fill it together
+      // (one step of 3e7 events in 40: 51 us per step when such a tile was
+      // added with float atomics, 20 in pieces; 300 pairs of 6000 events:
+      // 167 and 56 us).
+      const bool whole = !w.long_segments();
+      const uint32_t rest = w.E - done;
+      const uint32_t c = whole || rest < kBinPiece ? rest : kBinPiece;
+      uint32_t at0 = 0;
+      if (lane_id() == 0) at0 = atomicAdd(&s_n, c);
+      at0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)at0);
+      if (at0 + c > (uint32_t)kBinBuffer) {
+        // (the places from at0 on stay unused in this round)
+        if (lane_id() == 0) atomicMin(&s_n, at0);
+        waits = true;
+        continue;
+      }
+      auto put = [&](bool ok, uint32_t e, unsigned long long,
+                     unsigned long long r, float hj, uint32_t) {
+        if (!ok) return;
+        const uint32_t idx = acc_index((uint32_t)r, A.n_total);
+        const float v = hj * __uint_as_float((uint32_t)(r >> 32));
+        s_ev[at0 + (e - done)] =
+            ((unsigned long long)__float_as_uint(v) << 32) | idx;
+        atomicAdd(&s_cnt[idx >> kBinShift], 1u);
+      };
+      if (whole) {
+        w.spread(s_tab[threadIdx.x / 64], A.rec, put);
       } else {
-        uint32_t at0 = 0;
-        if (lane_id() == 0) at0 = atomicAdd(&s_n, w.E);
-        at0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)at0);
-        if (at0 + w.E > (uint32_t)kBinBuffer) {
-          // (the places from at0 on stay unused in this round)
-          if (lane_id() == 0) atomicMin(&s_n, at0);
-          waits = true;
-          continue;
-        }
-        w.emit(s_tab[threadIdx.x / 64], A.rec,
-               [&](bool ok, uint32_t e, unsigned long long,
-                   unsigned long long r, float hj, uint32_t) {
-                 if (!ok) return;
-                 const uint32_t idx = acc_index((uint32_t)r, A.n_total);
-                 const float v = hj * __uint_as_float((uint32_t)(r >> 32));
-                 s_ev[at0 + e] =
-                     ((unsigned long long)__float_as_uint(v) << 32) | idx;
-                 atomicAdd(&s_cnt[idx >> kBinShift], 1u);
-               });
+        w.template walk<true>(A.rec, done, done + c, put);
+        done += c;
+        if (done < w.E) continue;
+        done = 0;
       }
       loaded = false;
       wt += t.n_waves;

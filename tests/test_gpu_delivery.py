@@ -53,7 +53,9 @@ def state(ngpu, neuron, settings, steps):
 @pytest.mark.parametrize("n,n_src,k,slots", [
     (1000, 1, 1, 1), (1000, 7, 63, 2), (5000, 65, 129, 20),
     (20000, 3, 40000, 5),       # a pair of 28000 events
-    (40000, 300, 700, 64), (3000, 90, 500, 65)])
+    (40000, 300, 700, 64), (3000, 90, 500, 65),
+    (6000, 2000, 300, 1),       # wave tiles of many pairs, 12000 events
+    (9000, 33, 8200, 2)])       # pieces of a pair that end off a multiple
 def test_delivery_modes_agree(ngpu, n, n_src, k, slots):
     print("case delivery_modes", n, n_src, k, slots, flush=True)
     steps = min(slots, 12) + 6
