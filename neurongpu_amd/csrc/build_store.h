@@ -50,6 +50,13 @@ const char *TiledSumBound(const unsigned long long *trec, const uint32_t *off,
                           long long n_total, unsigned long long *bound,
                           float *max_w, void *stream);
 
+// Synapses onto every range of 2^shift accumulator entries (bin,
+// (port * n_total + target) >> shift): the host array cnt[0 .. nb-1].
+// Returns null on success or a static error message.
+const char *CountBinSynapses(const unsigned long long *rec,
+                             unsigned long long S, long long n_total,
+                             int shift, int nb, uint32_t *cnt, void *stream);
+
 // Synapse counts of the canonical store (device pointers): for nodes lo ..
 // hi-1, in_deg[t - lo] += synapses with target t, out_deg[s - lo] +=
 // synapses with source s, delay_cnt[d] += synapses with source in the range

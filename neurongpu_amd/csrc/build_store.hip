@@ -175,6 +175,26 @@ __global__ __launch_bounds__(kBoundBlock) void tile_bound(
   }
 }
 
+// Synapses per accumulator range, counted in LDS.
+__global__ __launch_bounds__(256) void bin_synapses(
+    const unsigned long long *rec, unsigned long long S, long long n_total,
+    int shift, int nb, uint32_t *cnt) {
+  extern __shared__ uint32_t s_cnt[];
+  for (int b = threadIdx.x; b < nb; b += 256) s_cnt[b] = 0u;
+  __syncthreads();
+  for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < S;
+       i += gridDim.x * 256ull) {
+    const uint32_t tp = (uint32_t)rec[i];
+    const unsigned long long a =
+        (unsigned long long)(tp >> kPortShift) * (unsigned long long)n_total +
+        (tp & kTargetMask);
+    atomicAdd(&s_cnt[a >> shift], 1u);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < nb; b += 256)
+    if (s_cnt[b]) atomicAdd(cnt + b, s_cnt[b]);
+}
+
 // Records of the tiled store: the entry within its tile in the low word
 // instead of the target and port.
 __global__ void gather_tiled(const uint32_t *idx, const unsigned long long *in,
@@ -444,6 +464,25 @@ const char *TiledSumBound(const unsigned long long *trec, const uint32_t *off,
     return "tiled bound failed";
   for (uint32_t t = 0; t < T; t++) *bound = std::max<unsigned long long>(*bound, h[t]);
   std::memcpy(max_w, &h[T], sizeof(float));
+  return nullptr;
+}
+
+const char *CountBinSynapses(const unsigned long long *rec,
+                             unsigned long long S, long long n_total,
+                             int shift, int nb, uint32_t *cnt,
+                             void *stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  const size_t bytes = (size_t)nb * sizeof(uint32_t);
+  DTmp<uint32_t> d(nb);
+  if (!d.p) return "out of device memory";
+  if (hipMemsetAsync(d.p, 0, bytes, stream) != hipSuccess)
+    return "hipMemsetAsync failed";
+  hipLaunchKernelGGL(bin_synapses, dim3(2048), dim3(256), bytes, stream, rec,
+                     S, n_total, shift, nb, d.p);
+  if (hipMemcpyAsync(cnt, d.p, bytes, hipMemcpyDeviceToHost, stream) !=
+          hipSuccess ||
+      hipStreamSynchronize(stream) != hipSuccess)
+    return "synapse count failed";
   return nullptr;
 }
 

@@ -362,7 +362,9 @@ class Engine {
   StepClock *StepClockNext() const { return d_clock.p + (clock_slot ^ 1); }
   void DropGraphs();
   StepClock HostClock() const;  // values of the next step
-  DBuf<uint32_t> d_bin_tot, d_bin_cstart, d_bin_meta;
+  DBuf<uint32_t> d_bin_tot, d_bin_cstart, d_bin_meta, d_bin_off;
+  std::vector<uint32_t> bin_syn;   // synapses onto each bin
+  long long bin_events = -1;       // size that d_bin_off divides
   DBuf<unsigned long long> d_bin_ev;
   DBuf<float> d_bin_part;
   // sets up the binned-delivery buffers; false if the network cannot use it

@@ -1928,7 +1928,8 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
         B.nb, [&](int b) -> uint32_t { return s_cnt[b]; },
         [&](int b, uint32_t first) {
           const uint32_t c = s_cnt[b];
-          s_to[b] = (c ? atomicAdd(&B.tot[(size_t)b * kBinStride], c) : 0u) -
+          s_to[b] = (c ? B.off[b] + atomicAdd(&B.tot[(size_t)b * kBinStride], c)
+                       : 0u) -
                     first;
           s_cnt[b] = first;
         },
@@ -1955,8 +1956,8 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
       const unsigned long long e = s_ev[j];
       const uint32_t idx = (uint32_t)e, b = idx >> kBinShift;
       const uint32_t pos = j + s_to[b];
-      if (pos < B.bin_cap)
-        B.ev[(size_t)b * B.bin_cap + pos] =
+      if (pos < B.off[b + 1])
+        B.ev[pos] =
             (e & 0xFFFFFFFF00000000ull) | (idx & (kBinLen - 1));
       else
         unsafeAtomicAdd(A.acc + idx, __uint_as_float((uint32_t)(e >> 32)));
@@ -1974,7 +1975,8 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
 // Events of bin b in its buffer.
 __device__ __forceinline__ uint32_t bin_events(const BinArgs &B, int b) {
   const uint32_t n = B.tot[(size_t)b * kBinStride];
-  return n < B.bin_cap ? n : B.bin_cap;
+  const uint32_t room = B.off[b + 1] - B.off[b];
+  return n < room ? n : room;
 }
 
 __global__ __launch_bounds__(kReduceBlock) void bin_reduce_kernel(BinArgs B,
@@ -2054,7 +2056,7 @@ __global__ __launch_bounds__(kReduceBlock) void bin_reduce_kernel(BinArgs B,
       k = w - s_c[b];
       nc = s_c[b + 1] - s_c[b];
     }
-    const unsigned long long *ev = B.ev + (size_t)b * B.bin_cap;
+    const unsigned long long *ev = B.ev + B.off[b];
     const uint32_t e_end = bin_events(B, b);
     const uint32_t e0 = k * ch;
     const uint32_t e1 = (e_end - e0 < ch) ? e_end : e0 + ch;

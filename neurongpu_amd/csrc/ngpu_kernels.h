@@ -378,12 +378,13 @@ struct BinArgs {
   uint32_t *tot;            // [nb][kBinStride] events of each bin, in the
                             // first element (0 between steps)
   uint32_t *cstart;         // [nb+1] first chunk of each bin
-  unsigned long long *ev;   // [nb][bin_cap] (index within bin, value bits)
+  unsigned long long *ev;   // (index within bin, value bits), bin b's from
+                            // off[b] on
+  const uint32_t *off;      // [nb+1] room of the bins; events beyond a
+                            // bin's are added with float atomics
   float *part;              // [chunk_cap][kBinLen] partial sums,
                             // chunk_cap = kReduceChunks + nb
   uint32_t *meta;           // [1] whether some bin has more than one chunk
-  uint32_t bin_cap;         // events beyond it in a bin are added with
-                            // float atomics
   int nb;                   // bins: ceil(acc_n / kBinLen)
   int grid;                 // blocks of the scatter
   long long acc_n;          // accumulator entries (ports x nodes)

@@ -6,6 +6,7 @@ the atomic delivery's sums bit for bit.
 """
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +78,41 @@ def test_delivery_modes_agree(ngpu, n, n_src, k, slots):
             assert sum(float(np.abs(w).sum()) for w in want) > 0.0
         for a, b in zip(want, got):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("targets", [100000, 3000])
+def test_binned_buffer_holds_the_synapses(ngpu, targets):
+    """1e7 synapses onto 25 accumulator ranges, evenly or (3000 targets) all
+    onto the first ranges of the two ports: the buffer of the binned mode
+    takes 8 bytes a synapse, and the sums are the atomic delivery's."""
+    print("case binned_buffer", targets, flush=True)
+    n, n_src, k = 100000, 100, 50000
+
+    def go(mode):
+        ngpu.ResetKernel()
+        ngpu.SetVerbosityLevel(0)
+        neuron = ngpu.Create("iaf_psc_exp", n)
+        gen = ngpu.Create("spike_generator", n_src)
+        for i in range(n_src):
+            ngpu.SetStatus([gen[i]], {"spike_times": [0.1 * (1 + i % 4)]})
+        for port in (0, 1):
+            ngpu.Connect(gen, ngpu.NodeSeq(neuron.i0, targets),
+                         {"rule": "fixed_total_number", "total_num": n_src * k},
+                         {"weight": 0.25, "delay": 0.2, "receptor": port})
+        ngpu.SetKernelStatus("delivery_mode", mode)
+        ngpu.SetSimTime(0.8)
+        ngpu.StartSimulation()
+        free = torch.cuda.mem_get_info()[0]
+        ngpu.SimulationStep()
+        used = free - torch.cuda.mem_get_info()[0]
+        for _ in range(7):
+            ngpu.SimulationStep()
+        ngpu.EndSimulation()
+        return used, [np.array(ngpu.GetNeuronVar(neuron.i0, n, v))
+                      for v in ("I_syn_ex", "I_syn_in")]
+
+    _, want = go(0)
+    used, got = go(1)
+    assert used < 8 * 2 * n_src * k + (64 << 20)
+    for a, b in zip(want, got):
+        assert a.any() and np.array_equal(a, b)
