@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kTB) void grad_kernel(PropTrainArgs A) {
   for (int r = 0; r < 16; r++) g2[r] = g1[r] = 0.0f;
   float gb2 = 0.0f, gw3 = 0.0f;         // of unit col, samples of this half
   float gb3 = 0.0f, loss = 0.0f;
-  const int tiles = (A.batch + kTile - 1) / kTile;
+  const int tiles = (int)(((uint32_t)A.batch + kTile - 1u) / kTile);
   // every wave of the block makes the same number of passes
   for (int t0 = blockIdx.x * kGradWaves; t0 < tiles;
        t0 += gridDim.x * kGradWaves) {
@@ -278,7 +278,7 @@ const char *LaunchPropTrainStep(const PropTrainArgs &a, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   if (a.batch <= 0) return "batch must be positive";
   // a wave per tile up to one block per CU
-  const int tiles = a.batch / kTile + (a.batch % kTile ? 1 : 0);
+  const int tiles = (int)(((uint32_t)a.batch + kTile - 1u) / kTile);
   int rows = tiles / kGradWaves + (tiles % kGradWaves ? 1 : 0);
   if (rows > kPropGradRows) rows = kPropGradRows;
   hipLaunchKernelGGL(grad_kernel, dim3(rows), dim3(kTB), 0, s, a);

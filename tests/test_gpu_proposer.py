@@ -244,3 +244,26 @@ def test_proposer_in_step_keeps_statistics(ngpu, settings):
     assert f_p < 0.02
     assert f_l <= 1.1 * f_p
     assert stages(c_learned) < stages(c_plain)
+
+
+def test_training_step_of_the_largest_batch(ngpu):
+    """A batch of 2^31 - 1 draws of the one logged sample: the loss and the
+    gradients (plain descent) of that sample alone.  A lane adds 65536 equal
+    losses, a wave 2^21 equal products, each sum's error at most n 2^-24."""
+    log("case largest_batch")
+    ngpu.SetRandomSeed(5)
+    x = np.zeros((1, ngpu.PROPOSER_SAMPLE), dtype=np.float32)
+    x[0, :7] = [0.3, -0.7, 1.1, 0.2, -0.4, 0.9, -2.0]
+    ngpu.ProposerSetSamples(x)
+    w0 = ngpu.ProposerGetWeights()
+    one = ngpu.ProposerTrain(1, batch=1, lr=0.5, adam=False)
+    d1 = ngpu.ProposerGetWeights() - w0
+    ngpu.ProposerSetWeights(w0)
+    most = ngpu.ProposerTrain(1, batch=2 ** 31 - 1, lr=0.5, adam=False)
+    d2 = ngpu.ProposerGetWeights() - w0
+    log("loss", one, most)
+    assert one > 0.0 and abs(most - one) <= (2.0 ** -8 + 1e-5) * one
+    # (w0 + d rounds to the weights' last bit)
+    assert np.all(np.abs(d2 - d1) <= 0.126 * np.abs(d1) +
+                  2.0 ** -23 * np.abs(w0))
+    assert np.count_nonzero(d1) > 100
