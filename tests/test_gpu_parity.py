@@ -448,7 +448,8 @@ def test_ensemble_routing_matches_instances_alone(ngpu):
 
 @pytest.mark.parametrize("settings", [
     {"rk5_two_pass": 0},
-    {"rk5_budget": 3, "rk5_pass2_grid": 64},
+    {"rk5_budget": 3, "rk5_pass2_grid": 64},   # (one launch a step)
+    {"rk5_budget": 3, "rk5_pass2_grid": 64, "fuse_delivery": 0},
     {"delivery_grid": 256, "delivery_tile_max": 8, "fuse_delivery": 0},
     {"delivery_grid": 4096, "delivery_tile_max": 1},
     {"delivery_mode": 1},

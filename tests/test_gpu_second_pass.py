@@ -36,11 +36,13 @@ def spec(ports, uniform, tol=1e-6):
          "rk5": {"rk5_tol": tol}}]}
 
 
-def run(ngpu, sp, settings):
+def run(ngpu, sp, settings, ms=60.0, change=()):
     groups, _ = wl.build_from_spec(ngpu, sp)
+    for node, name, val in change:
+        ngpu.SetStatus([node], {name: val})
     ngpu.SetKernelStatus(settings)
     ngpu.ActivateSpikeCount(groups[0])
-    ngpu.Simulate(60.0)
+    ngpu.Simulate(ms)
     out = [np.array(ngpu.GetNeuronVar(0, N, v))
            for v in ("V_m", "w", "g", "g1")]
     out.append(np.array(ngpu.GetNeuronIntVar(0, N, "spike_count")))
@@ -51,9 +53,9 @@ def run(ngpu, sp, settings):
 @pytest.mark.parametrize("uniform", [True, False])
 @pytest.mark.parametrize("ports", [1, 2, 3, 4])
 def test_second_pass_layouts(ngpu, ports, uniform):
-    """Grids of 256 blocks (every list fits the quads), 1 block (64 quads:
-    longer lists run on whole waves first), and binned steps, where the pass
-    overlaps the next step; 4 ports keep one lane per neuron."""
+    """Up to 3 ports these steps run in one launch (whatever the budget and
+    the second pass's grid), and binned, where the pass overlaps the next
+    step; 4 ports run in two passes, with one lane per neuron."""
     print("case second_pass", ports, uniform, flush=True)
     sp = spec(ports, uniform)
     want = run(ngpu, sp, {"rk5_two_pass": 0})
@@ -68,6 +70,133 @@ def test_second_pass_layouts(ngpu, ports, uniform):
             assert np.array_equal(a, b)
         # the same attempts, accepted and rejected
         assert got[5] == want[5]
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ports", [1, 2, 3])
+def test_second_pass_of_a_large_network(ngpu, ports, uniform):
+    """The second pass in the launch of the delivery, as networks of more
+    than 65536 neurons run it (here with silent ones beside the spiking):
+    256 blocks (every list fits the quads), 1 block (64 quads; in the first
+    step, which starts at a hundredth of the time step, all 700 neurons are
+    listed and run on whole waves first), a budget of 3 attempts."""
+    print("case second_pass_large", ports, uniform, flush=True)
+    sp = spec(ports, uniform)
+    sp["groups"].append({"model": "iaf_psc_exp", "n": 65536})
+    want = run(ngpu, sp, {"rk5_two_pass": 0, "delivery_mode": 0})
+    assert want[4].sum() > 2 * N
+    for st in ({"rk5_pass2_grid": 256}, {"rk5_pass2_grid": 1},
+               {"rk5_pass2_grid": 256, "rk5_budget": 3},
+               {"rk5_pass2_grid": 1, "rk5_budget": 3}):
+        print("  settings", st, flush=True)
+        got = run(ngpu, sp, dict(st, delivery_mode=0))
+        for a, b in zip(want[:5], got[:5]):
+            assert np.array_equal(a, b)
+        assert got[5] == want[5]
+        # two launches a step: first pass; second pass with the delivery
+        ngpu.SetKernelTiming(1)
+        ngpu.Simulate(0.5)
+        kinds = ngpu.GetKernelTimes()
+        ngpu.SetKernelTiming(0)
+        assert kinds["aeif_rk5_pass2"][1] == kinds["aeif_rk5"][1] == 5
+        assert "delivery" not in kinds
+
+
+NAN, INF = float("nan"), float("inf")
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ports", [1, 2, 3])
+def test_neurons_with_invalid_state(ngpu, ports, uniform):
+    """NaN and infinite membrane potentials, adaptation currents and
+    conductances in some neurons of a wave: the same bits (any NaN as NaN),
+    attempts and forced accepts in every form of the step."""
+    print("case invalid_state", ports, uniform, flush=True)
+    sp = spec(ports, uniform)
+    odd = [(3, "V_m", NAN), (70, "w", NAN), (71, "g", [NAN] * ports),
+           (72, "g1", [NAN] * ports), (200, "V_m", INF),
+           (201, "V_m", -INF), (264, "w", INF), (265, "w", -INF),
+           (266, "g", [INF] * ports), (267, "g1", [INF] * ports),
+           (N - 1, "g1", [0.0] * (ports - 1) + [NAN])]
+    want = run(ngpu, sp, {"rk5_two_pass": 0}, 5.0, odd)
+    assert np.isnan(want[0][[3, 72, N - 1]]).all()
+    for st in ({}, {"fuse_delivery": 0}, {"delivery_mode": 1}):
+        print("  settings", st, flush=True)
+        got = run(ngpu, sp, st, 5.0, odd)
+        for a, b in zip(want[:4], got[:4]):
+            assert np.array_equal(a, b, equal_nan=True)
+        assert np.array_equal(want[4], got[4])
+        assert got[5] == want[5]
+
+
+@pytest.mark.parametrize("ports", [1, 2, 3])
+def test_attempt_cap(ngpu, ports):
+    """A neuron whose error is NaN at a minimum step of 1e-6 time steps
+    reaches the cap of attempts and gives the time step up."""
+    print("case attempt_cap", ports, flush=True)
+    sp = spec(ports, True)
+    sp["groups"][0]["rk5"]["h_min_rel"] = 1e-6
+    odd = [(i, "g1", [0.0] * (ports - 1) + [NAN]) for i in (5, 300, N - 1)]
+    want = run(ngpu, sp, {"rk5_two_pass": 0}, 0.3, odd)
+    assert want[5]["rk5_rejected"] > 3 * 3 * 40000
+    assert want[5]["rk5_accepted"] < 3 * 3 * 60000 + 3 * N * 100
+    for st in ({}, {"fuse_delivery": 0}, {"delivery_mode": 1}):
+        print("  settings", st, flush=True)
+        got = run(ngpu, sp, st, 0.3, odd)
+        for a, b in zip(want[:4], got[:4]):
+            assert np.array_equal(a, b, equal_nan=True)
+        assert np.array_equal(want[4], got[4])
+        assert got[5] == want[5]
+
+
+@pytest.mark.parametrize("h_min", [1e-3, 1e-6])
+@pytest.mark.parametrize("ports", [1, 3])
+@pytest.mark.parametrize("model", ["aeif_psc_alpha", "aeif_psc_exp"])
+def test_psc_neurons_with_invalid_state(ngpu, model, ports, h_min):
+    """The same for the current-based models against the FP32 oracle; at the
+    smaller minimum step the NaN errors reach the cap."""
+    print("case psc_invalid", model, ports, h_min, flush=True)
+    n, steps = 70, (30 if h_min == 1e-3 else 2)
+    rng = np.random.default_rng(ports)
+    last = "I1_syn" if model == "aeif_psc_alpha" else "I_syn"
+    sp = {"seed": 7, "groups": [
+        {"model": model, "n": n, "n_port": ports,
+         "params": {"I_e": rng.uniform(700.0, 1500.0, n), "t_ref": 0.5,
+                    "V_peak": 0.0},
+         "vars": {"V_m": rng.uniform(-70.0, -50.0, n).astype(np.float32)},
+         "rk5": {"h_min_rel": h_min}}]}
+    odd = [(5, last, NAN), (66, last, NAN)]
+    if h_min == 1e-3:
+        odd += [(0, "V_m", NAN), (1, "w", NAN), (2, "I_syn", INF),
+                (63, "V_m", INF), (64, "V_m", -INF), (65, "w", INF),
+                (67, "w", -INF), (68, last, -INF)]
+    groups, _ = nb.build_engine(ngpu, sp)
+    net, og = nb.build_oracle(sp, "f32")
+    for name in {v for _, v, _ in odd}:
+        vals = np.array(og[0].get(name), dtype=np.float64)
+        for i, v, x in odd:
+            if v == name:
+                vals[i] = x
+                ngpu.SetStatus([i], {v: x if v in ("V_m", "w")
+                                     else [x] * ports})
+        og[0].set(name, vals)
+    ngpu.ActivateSpikeCount(groups[0])
+    ngpu.Simulate(0.1 * steps)
+    net.run(steps)
+    for v in ("V_m", "w"):
+        assert np.array_equal(np.array(ngpu.GetNeuronVar(0, n, v)),
+                              np.array(og[0].get(v), dtype=np.float32),
+                              equal_nan=True)
+    cur = np.array(ngpu.GetNeuronVar(0, n, "I_syn"))
+    for q in range(ports):
+        assert np.array_equal(cur.reshape(n, ports)[:, q],
+                              np.array(og[0].get("I_syn", q),
+                                       dtype=np.float32), equal_nan=True)
+    count = np.array(ngpu.GetNeuronIntVar(0, n, "spike_count"))
+    _, node, times = net.spikes()
+    want = np.zeros(n, int)
+    np.add.at(want, np.asarray(node, int), np.asarray(times, int))
+    assert np.array_equal(count, want)
 
 
 @pytest.mark.parametrize("n", [1, 70, 300])
