@@ -50,6 +50,72 @@ def test_range_and_list_reads(ngpu, model, ports):
         assert seen > 0      # some neuron was refractory at a read
 
 
+# parameters with a value per neuron, and per port and half of the neurons
+SCAL = {"aeif_cond_beta": ["C_m", "den_delay"],
+        "aeif_psc_exp": ["C_m", "V_peak"],
+        "izhikevich_cond_beta": ["a", "d"]}
+PORT = {"aeif_cond_beta": {"E_rev": (0.0, -85.0), "tau_decay": (2.0, 5.0)},
+        "aeif_psc_exp": {"tau_syn": (2.0, 1.0, 5.0)},
+        "izhikevich_cond_beta": {"tau_rise": (1.5,), "E_rev": (-3.0,)}}
+DRIVE = {"aeif_cond_beta": 900.0, "aeif_psc_exp": 900.0,
+         "izhikevich_cond_beta": 30.0}
+
+
+@pytest.mark.parametrize("model", list(SCAL))
+def test_refractory_count_and_parameters_by_value(ngpu, model):
+    """The refractory count step by step: t_ref / dt after a spike (one less
+    where the spike was not in the step's last RK5 step), then one less per
+    step; the other parameters as they were set."""
+    print("case readback_values", model, flush=True)
+    n, R, ports = 5000, 15, len(next(iter(PORT[model].values())))
+    ngpu.ResetKernel()
+    ngpu.SetVerbosityLevel(0)
+    ns = ngpu.Create(model, n, ports)
+    ngpu.SetStatus(ns, {"t_ref": 0.1 * R, "I_e": DRIVE[model]})
+    ngpu.SetStatus(ns, {"V_m": {"array": np.linspace(-45.0, -65.0, n)
+                                .astype(np.float32)}})
+    scal = {}
+    for k, name in enumerate(SCAL[model]):
+        base = np.array(ngpu.GetNeuronParam(0, n, name), dtype=np.float32)
+        scal[name] = (base + np.arange(n) % 7 * 0.1).astype(np.float32)
+        ngpu.SetStatus(ns, {name: {"array": scal[name]}})
+    port = {}
+    for name, vals in PORT[model].items():
+        other = [v + 0.5 for v in vals]
+        ngpu.SetStatus(ns, {name: list(vals)})
+        ngpu.SetStatus(ns[n // 2:n], {name: other})
+        port[name] = np.repeat([vals, other], n // 2, axis=0)
+    ngpu.ActivateSpikeCount(ns)
+    ngpu.SetSimTime(25.0)
+    ngpu.StartSimulation()
+    refr, count = np.zeros(n), np.zeros(n, int)
+    at_end = 0
+    for step in range(250):
+        ngpu.SimulationStep()
+        r = np.array(ngpu.GetNeuronParam(0, n, "refractory_step"))
+        c = np.array(ngpu.GetNeuronIntVar(0, n, "spike_count"))
+        spk = c > count
+        assert np.array_equal(r[~spk], np.maximum(refr - 1.0, 0.0)[~spk])
+        assert np.isin(r[spk], (R, R - 1)).all()
+        at_end += int((r[spk] == R).sum())
+        refr, count = r, c
+        if step % 50 == 0:
+            for name in scal:
+                assert np.array_equal(
+                    np.array(ngpu.GetNeuronParam(0, n, name),
+                             dtype=np.float32), scal[name])
+    ngpu.EndSimulation()
+    assert count[0] > 0 and count[-1] > 0 and at_end < count.sum()
+    for name in ngpu.GetPortParamNames(0):
+        whole = np.array(ngpu.GetNeuronParam(0, n, name)).reshape(n, ports)
+        nodes = [0, n // 2 - 1, n // 2, 4096, n - 1]
+        assert np.array_equal(
+            whole[nodes],
+            np.array(ngpu.GetNeuronPtParam(nodes, name)).reshape(-1, ports))
+        if name in port:
+            assert np.array_equal(whole, port[name].astype(np.float32))
+
+
 def test_plastic_weights_by_source_range(ngpu):
     print("case readback plastic", flush=True)
     sp = wl.c3_spec(0.005, k=50, w_p=0.6)
