@@ -745,18 +745,6 @@ __device__ __forceinline__ void aeif_quad_finish(
            });
 }
 
-// The launch's AeifArgs (its first parameter), read again from the argument
-// segment through a pointer that the compiler cannot trace: values loaded
-// from it are neither loaded before this point nor kept in registers across
-// it.  The second pass has far more arguments than scalar registers; read up
-// front they cost its empty launches a microsecond of loads and spills.
-__device__ __forceinline__ const AeifArgs &late_args() {
-  auto p = (const __attribute__((address_space(4))) AeifArgs *)
-      __builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return *(const AeifArgs *)p;
-}
-
 // Second pass: the listed neurons, run to the end of the step.  The
 // sub-lists are concatenated (prefix over their counts, in LDS) and lane g
 // of the grid takes entries g, g + G, ...; a lane moves on to its next
@@ -807,7 +795,7 @@ __device__ __forceinline__ void aeif_pass2_body(const AeifArgs &A0,
   // With the proposer every attempt runs in the lane loop below, where late
   // arguments would be read again after each store: it takes them as passed
   // (1e6 spiking neurons, tol 1e-6, 100 ms: 134 -> 132 ms in the mean).
-  const AeifArgs &A = PROP ? A0 : late_args();
+  const AeifArgs &A = PROP ? A0 : late_args<AeifArgs>();
   // the pass is a few long dependent chains: its waves issue first when
   // they share a SIMD with the first pass or the delivery
   if (CU) __builtin_amdgcn_s_setprio(3);
@@ -893,8 +881,9 @@ __device__ __forceinline__ void aeif_pass2_body(const AeifArgs &A0,
     if constexpr (kQuad) {
       if (quads && __popcll(running) <= kQuadsPerWave &&
           __ballot(j < total) == 0ull) {
-        aeif_quad_finish<P, UNI>(late_args(), sn, x1, have, i, y, scal, x, h, refr, nsp,
-                                 n_att, need_k1, n_acc, n_rej);
+        aeif_quad_finish<P, UNI>(late_args<AeifArgs>(), sn, x1, have, i, y,
+                                 scal, x, h, refr, nsp, n_att, need_k1, n_acc,
+                                 n_rej);
         break;
       }
     }
@@ -1082,7 +1071,7 @@ __device__ __forceinline__ void aeif_step_body(const AeifArgs &A,
     const unsigned long long running = lanes_where(run);
     if (running == 0ull) break;
     if (!first && __popcll(running) <= kQuadsPerWave) {
-      aeif_quad_finish<P, UNI>(late_args(), sn, x1, run, i, y, scal, x, h,
+      aeif_quad_finish<P, UNI>(late_args<AeifArgs>(), sn, x1, run, i, y, scal, x, h,
                                refr, nsp, n_att, need_k1, n_acc, n_rej);
       break;
     }

@@ -416,5 +416,19 @@ __device__ __forceinline__ void rk5_count_one(unsigned long long *cnt,
   }
 }
 
+// The launch's first argument, read again from the argument segment through
+// a pointer that the compiler cannot trace: values loaded from it are
+// neither loaded before this point nor kept in registers across it.  The RK5
+// kernels have far more arguments than scalar registers; read up front they
+// cost the second pass's empty launches a microsecond of loads and spills,
+// and the models of rk5_models.hip 90 spilled registers.
+template <class T>
+__device__ __forceinline__ const T &late_args() {
+  auto p = (const __attribute__((address_space(4))) T *)
+      __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const T *)p;
+}
+
 }  // namespace
 }  // namespace ngpu
