@@ -752,7 +752,8 @@ __device__ __forceinline__ void aeif_quad_finish(
 // neurons need different numbers of attempts, and waves beyond the list
 // end exit at once.
 // PROP: the learned proposer's inference is compiled in (its weights in
-// LDS, the MFMA registers); without it the pass keeps its occupancy.
+// LDS, the MFMA registers); without it the pass keeps its occupancy.  Used
+// for the sample log as well, with or without the proposer.
 template <int P, bool UNI, bool PROP, bool CU>
 __device__ __forceinline__ void aeif_pass2_body(const AeifArgs &A0,
                                                 uint32_t vblock,
@@ -792,9 +793,10 @@ __device__ __forceinline__ void aeif_pass2_body(const AeifArgs &A0,
                                                               : 64u;
   const uint32_t per_block = per_wave * (kBlock / 64);
   if (vblock * per_block >= total) return;  // whole block beyond the list
-  // With the proposer every attempt runs in the lane loop below, where late
-  // arguments would be read again after each store: it takes them as passed
-  // (1e6 spiking neurons, tol 1e-6, 100 ms: 134 -> 132 ms in the mean).
+  // With the proposer or its sample log every attempt runs in the lane loop
+  // below, where late arguments would be read again after each store: it
+  // takes them as passed (1e6 spiking neurons, tol 1e-6, 100 ms: 134 -> 132
+  // ms in the mean).
   const AeifArgs &A = PROP ? A0 : late_args<AeifArgs>();
   // the pass is a few long dependent chains: its waves issue first when
   // they share a SIMD with the first pass or the delivery
@@ -2422,7 +2424,10 @@ void launch_aeif_pass2_p(const AeifArgs &a, const DeliveryArgs *d,
       return;
     }
   }
-  if (a.prop_pk && kProp) {
+  // The sample log works on whole lanes too: the instance whose arguments
+  // stay in registers (1e5 spiking neurons with the log on: 122 us per step
+  // in the one made for quads, 114 in this one)
+  if ((a.prop_pk || a.prop_log) && kProp) {
     if (a.uniform)
       launch_pass2_v<P, true, kProp, false>(a, d, grid2, d_grid, s);
     else
