@@ -476,6 +476,9 @@ class Engine {
                    long long it_local);
   void EnsureHostCSR();
   void BuildDeviceStore();
+  // Range reads since the plastic weights last changed, in records that
+  // copying them costs (SourceRangeRows)
+  unsigned long long range_cost = 0;
   // the rows of sources s0 .. s0+n-1 in three copies: base[0..n] (offsets
   // into rec, relative to base[0]), seg[(D+1)*i ..] and rec; with sg also
   // their synapse groups (empty in a network without plastic synapses)

@@ -141,3 +141,25 @@ def test_plastic_weights_by_source_range(ngpu):
     for key in part:
         assert np.array_equal(part[key], after[key][sel])
     assert np.any(after["weight"] != before["weight"])
+
+
+def test_many_plastic_queries(ngpu):
+    """One query per source, again after more steps: the first ones read
+    their range from the device, the later ones the host copy that they are
+    worth by then; both as one query of all sources."""
+    print("case readback many", flush=True)
+    sp = wl.c3_spec(0.005, k=50, w_p=0.6)
+    wl.build_from_spec(ngpu, sp)
+    n_e = sp["populations"][0][1]
+    ns = ngpu.NodeSeq(0, n_e)
+    weights = []
+    for _ in range(2):
+        ngpu.Simulate(100.0)
+        parts = [ngpu.GetConnectionArrays(source=ns[i:i + 1], target=ns)
+                 for i in range(n_e)]
+        whole = ngpu.GetConnectionArrays(source=ns, target=ns)
+        for key in whole:
+            assert np.array_equal(whole[key],
+                                  np.concatenate([p[key] for p in parts]))
+        weights.append(whole["weight"])
+    assert np.any(weights[0] != weights[1])
