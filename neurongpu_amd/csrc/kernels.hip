@@ -1844,17 +1844,18 @@ inline size_t scatter_lds_bytes(int D, int nb) {
 // enumerated twice (counts, a scan over the blocks, then the events at
 // their final places).
 __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
-    DeliveryArgs A0, BinArgs B) {
+    BinArgs B0, DeliveryArgs A0) {
   const DeliveryArgs A = clocked(A0);
+  const int nb = B0.nb;
   unsigned long long *s_ev = reinterpret_cast<unsigned long long *>(s_dyn);
   uint32_t *s_pre = s_dyn + 2 * kBinBuffer;
   uint32_t *s_cnt = s_pre + A.D + 1;   // events of the round per bin; then
                                        // the next one's place in the order
-  uint32_t *s_to = s_cnt + B.nb;       // from that place to the bin's buffer
+  uint32_t *s_to = s_cnt + nb;       // from that place to the bin's buffer
   __shared__ PairTable<true> s_tab[kBinBlock / 64];
   __shared__ uint32_t s_part[kBinBlock / 64];
   __shared__ uint32_t s_n;             // events in the buffer
-  for (int b = threadIdx.x; b < B.nb; b += kBinBlock) s_cnt[b] = 0u;
+  for (int b = threadIdx.x; b < nb; b += kBinBlock) s_cnt[b] = 0u;
   if (threadIdx.x == 0) s_n = 0u;
   const uint32_t total = delivery_prologue<kBinBlock>(
       A, blockIdx.x, s_pre, reinterpret_cast<uint32_t *>(s_tab));
@@ -1919,15 +1920,20 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
     }
     const int more = __syncthreads_or(waits ? 1 : 0);
     // reserve the round's runs in the bins' buffers
+    // (read here: through the enumeration they would be spilled)
+    const BinArgs &L = late_args<BinArgs>();
+    uint32_t *const tot = L.tot;
+    const uint32_t *const off = L.off;
+    unsigned long long *const out = L.ev;
     int full = 0;                      // some run leaves its bin's room
     (void)block_scan_excl<kBinBlock>(
-        B.nb, [&](int b) -> uint32_t { return s_cnt[b]; },
+        nb, [&](int b) -> uint32_t { return s_cnt[b]; },
         [&](int b, uint32_t first) {
           const uint32_t c = s_cnt[b];
           uint32_t to = 0u;
           if (c) {
-            to = B.off[b] + atomicAdd(&B.tot[(size_t)b * kBinStride], c);
-            full |= to + c > B.off[b + 1];
+            to = off[b] + atomicAdd(&tot[(size_t)b * kBinStride], c);
+            full |= to + c > off[b + 1];
           }
           s_to[b] = to - first;
           s_cnt[b] = first;
@@ -1950,14 +1956,14 @@ __global__ __launch_bounds__(kBinBlock) void bin_scatter_kernel(
       if (k * kBinBlock + threadIdx.x < n)
         s_ev[atomicAdd(&s_cnt[(uint32_t)ev[k] >> kBinShift], 1u)] = ev[k];
     __syncthreads();
-    for (int b = threadIdx.x; b < B.nb; b += kBinBlock) s_cnt[b] = 0u;
+    for (int b = threadIdx.x; b < nb; b += kBinBlock) s_cnt[b] = 0u;
     auto leave = [&](bool room) {
       for (uint32_t j = threadIdx.x; j < n; j += kBinBlock) {
         const unsigned long long e = s_ev[j];
         const uint32_t idx = (uint32_t)e, b = idx >> kBinShift;
         const uint32_t pos = j + s_to[b];
-        if (room || pos < B.off[b + 1])
-          B.ev[pos] = (e & 0xFFFFFFFF00000000ull) | (idx & (kBinLen - 1));
+        if (room || pos < off[b + 1])
+          out[pos] = (e & 0xFFFFFFFF00000000ull) | (idx & (kBinLen - 1));
         else
           unsafeAtomicAdd(A.acc + idx, __uint_as_float((uint32_t)(e >> 32)));
       }
@@ -2659,7 +2665,7 @@ void LaunchDeliveryBinned(const DeliveryArgs &a, const BinArgs &b,
     lds_attr = true;
   }
   hipLaunchKernelGGL(bin_scatter_kernel, dim3(b.grid), dim3(kBinBlock),
-                     scatter_lds_bytes(a.D, b.nb), s, a, b);
+                     scatter_lds_bytes(a.D, b.nb), s, b, a);
   hipLaunchKernelGGL(bin_reduce_kernel, dim3(reduce_grid), dim3(kReduceBlock),
                      sizeof(uint32_t) * ((size_t)b.nb + 1), s, b, a.acc);
   // Many bins of about equal size leave nothing to sum (128 blocks: the
