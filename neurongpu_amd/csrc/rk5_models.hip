@@ -362,7 +362,7 @@ __global__ __launch_bounds__(kBlock) void rk5_model_kernel(Rk5ModelArgs A) {
   // The wave's finished neurons together: whole cache lines, one append.
   // The quads follow behind the loop, where nothing of it is live (5e5
   // neurons of aeif_psc_exp, 2 ports: 144 registers and 20.4 us per step
-  // with both inside the loop, 89 and 17.8).
+  // with both inside the loop, 89 and 18).
   const Rk5ModelArgs &L = late_args<Rk5ModelArgs>();
   const bool done = active && !run;
   if (done) {
